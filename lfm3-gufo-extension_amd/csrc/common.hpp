@@ -102,9 +102,10 @@ inline bool BufferFits(std::size_t bytes) { return bytes < std::size_t(kOutOfRan
 __device__ __forceinline__ BufferResource MakeBuffer(const void* base, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, int(bytes), kBufferWord3);
 }
-__device__ __forceinline__ uint4 LoadB128(BufferResource res, unsigned offset) {
+__device__ __forceinline__ uint4 LoadB128(BufferResource res, unsigned offset,
+                                          unsigned scalar_offset = 0) {
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(res, offset, 0, 0);
+  const u4 v = __builtin_amdgcn_raw_buffer_load_b128(res, offset, scalar_offset, 0);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 __device__ __forceinline__ float4 LoadF4(BufferResource res, unsigned offset) {
@@ -120,6 +121,23 @@ __device__ __forceinline__ unsigned LoadB32(BufferResource res, unsigned offset)
 // sees them.
 constexpr int WaitVm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 constexpr int kWaitLgkm0 = 15 | (3 << 14) | (7 << 4);
+
+// A block barrier that orders the compiler only: vector memory operations in
+// flight stay in flight, and the caller waits for its own LDS operations.
+__device__ __forceinline__ void BlockBarrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Block b of a launch -> work item, XCD-major: blocks are dispatched to
+// the 8 XCDs round robin (b % 8), so XCD x gets the consecutive items
+// [first(x), first(x) + count(x)); items sharing weight rows are adjacent,
+// so their tiles come from HBM once per XCD and then from its L2.
+__device__ __forceinline__ int XcdMajorItem(int b, int blocks) {
+  const int q = blocks / 8, rem = blocks % 8, x = b % 8, i = b / 8;
+  return (x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + i;
+}
 
 // Per-component select (a select of whole vectors in a register array can
 // become a select of addresses into scratch memory).

@@ -1405,13 +1405,15 @@ void RunPrompt(lfm3_model& m, lfm3_session& se, const std::vector<ChunkPart>& in
                                cols, s));
   };
   // Float-weight models run every projection through the exact float GEMV
-  // over all rows at once (hip/ops.hip:2230-2249 for float tensors).
+  // over all rows at once (hip/ops.hip:2230-2249 for float tensors), in K
+  // parts where the consumer adds them.
   const std::uint32_t mfma_rows = m.exact ? 0xffffffffu : kPromptRows;
   const auto gemv = [&](const Matrix& w, const float* in, std::uint32_t ldx, float* y,
-                        std::uint32_t ldy, std::uint32_t rows, bool swiglu) {
+                        std::uint32_t ldy, std::uint32_t rows, bool swiglu,
+                        std::uint32_t parts = 1) {
     if (w.exact) {
       CheckStatus(lfm3_float_gemv(w.type, w.codes.p, swiglu ? F : w.rows, w.cols, in, ldx, y,
-                                  ldy, rows, 1, swiglu ? 1 : 0, s));
+                                  ldy, rows, parts, swiglu ? 1 : 0, s));
       return;
     }
     for (std::uint32_t r = 0; r < rows; r += kMaxBatch) {
@@ -1446,8 +1448,10 @@ void RunPrompt(lfm3_model& m, lfm3_session& se, const std::vector<ChunkPart>& in
                            bool single) -> std::uint32_t {
     const std::uint32_t first = n - rows;
     if (rows < mfma_rows) {
-      gemv(w, z + std::size_t(first) * H, H, y, ldy, rows, false);
-      return 1;
+      const std::uint32_t parts =
+          w.exact && !single ? lfm3_bf16_gemv_parts(w.rows, w.cols, rows) : 1;
+      gemv(w, z + std::size_t(first) * H, H, y, ldy, rows, false, parts);
+      return parts;
     }
     if (!single)
       return gemm(w, first, rows, y, ldy);
@@ -1459,8 +1463,9 @@ void RunPrompt(lfm3_model& m, lfm3_session& se, const std::vector<ChunkPart>& in
   const auto dense = [&](const Matrix& w, const float* in, std::uint32_t ldx,
                          std::uint32_t rows, const unsigned* rmax) -> std::uint32_t {
     if (rows < mfma_rows) {
-      gemv(w, in, ldx, out, H, rows, false);
-      return 1;
+      const std::uint32_t parts = w.exact ? lfm3_bf16_gemv_parts(w.rows, w.cols, rows) : 1;
+      gemv(w, in, ldx, out, H, rows, false, parts);
+      return parts;
     }
     halves(in, ldx, rmax, rows, w.cols);
     return gemm(w, 0, rows, out, H);

@@ -20,11 +20,14 @@
 // most 3 bits; an F32 weight splits like the inputs. So the 3 x (1, 2 or
 // 3) MFMAs per 32-column block give the exact products of the weights
 // with the FP32 inputs; only the FP32 accumulation order differs from a
-// scalar loop. A block owns up to 16 tokens (A rows), RT row tiles and,
-// per wave, a contiguous range of column blocks; the waves' sums meet in
-// LDS and add in wave order.
+// scalar loop. Two kernels take these products. FloatGemvKernel (decode
+// rows, up to 16 tokens a block): RT row tiles a block and, per wave, a
+// contiguous range of column blocks; the waves' sums meet in LDS and add in
+// wave order. FloatGemmKernel (prompt rows): a block owns 64 tokens and
+// splits their inputs once for all of its weight rows.
 #include <cmath>
 #include <cstring>
+#include <utility>
 
 #include "common.hpp"
 #include "internal.hpp"
@@ -222,6 +225,303 @@ __launch_bounds__(kThreads) __global__
   }
 }
 
+// f(0), f(1), .., f(N - 1) with constant indices.
+template<int N, class F>
+__device__ __forceinline__ void Unroll(F f) {
+  [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) {
+    (f(std::integral_constant<int, I>{}), ...);
+  }(std::make_integer_sequence<int, N>{});
+}
+
+// y[p][t][r] for 16 TT tokens and 16 RT (8 / KG) weight rows a block, one K
+// part p of `parts`: the prompt rows' products (64 tokens; 32 when there are
+// no more).
+//
+// What bounds it: a decode-shaped block (16 tokens) reads every weight once
+// per 16 tokens and splits every input once per 16 RT rows, which left the
+// 512-token BF16 gate/up product (2 x 7680 x 2048) at 277-318 us; its 3 MFMAs
+// per tile, token group and 32 columns take 39 us at the matrix peak. This
+// kernel takes 79-83 us (410 TFLOP/s, 1.2 PFLOP/s of MFMAs), the down product
+// 49 us against 236, F16 gate/up 170 against 358, F32 209 against 565; what is
+// left is LDS latency at two waves a SIMD. A step of 128
+// columns is split once per block into operand order in LDS (each lane's 16
+// bytes at its own slot: no bank conflicts either way), double buffered, one
+// barrier a step; each wave owns its weight rows, read straight into
+// registers (the tiles are in operand order), so a weight byte enters a CU
+// once per 64 tokens. The eight waves are KG groups along K times 8 / KG
+// along the rows (256 rows a BF16 block when that fills the CUs; fewer rows
+// and more K groups when it does not); the groups' sums meet in LDS.
+//
+// Every four column blocks are a segment: the products of the inputs' mid and
+// lo parts first, then the hi parts', from zero, so that the small terms are
+// not rounded at the size of the large ones; the finished segments add in K
+// order. (A single chain over K = 2048 doubled the decode kernel's distance
+// to float64.) The formats in several parts keep the small products apart.
+constexpr int kStepKb = 4;  // column blocks a step
+
+template<int RT, int KG, int TT, bool kSwiGLU, int WF>
+__launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void FloatGemmKernel(const uint4* __restrict__ tiles, int row_tiles, int nkb,
+                                const float* __restrict__ x, int ldx, int batch,
+                                float* __restrict__ y, int ldy, int out_rows, int row_blocks,
+                                int token_blocks, int parts, std::size_t part_stride) {
+  constexpr int NW = WordsOf(WF), NP = PartsOf(WF);
+  constexpr int RG = kWaves / KG;          // waves along the rows
+  constexpr int kMine = kStepKb / KG;      // column blocks of a step a wave takes
+  constexpr int kBufs = KG == 1 ? kMine : 2 * kMine;  // weight buffers
+  constexpr int kAhead = KG == 4 ? 2 : 1;  // steps the inputs are loaded ahead
+  constexpr int kPairs = kStepKb * TT / kWaves;  // (column block, group) pairs a wave stages
+  static_assert(kMine >= 1 && kPairs * kWaves == kStepKb * TT);
+  constexpr int kStage = kStepKb * TT * 3 * 64;  // uint4 of one stage
+  constexpr int kRed = KG > 1 ? kWaves * RT * TT * 64 : 0;
+  __shared__ uint4 s_mem[2 * kStage > kRed ? 2 * kStage : kRed];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, m = lane & 15;
+  const int kg = wave / RG, rg = wave % RG;
+  const int item = XcdMajorItem(blockIdx.x, gridDim.x);
+  const int tb = item % token_blocks, rb = (item / token_blocks) % row_blocks;
+  const int part = item / (token_blocks * row_blocks);
+  const int tile0 = (rb * RG + rg) * RT, tok0 = tb * 16 * TT;
+  const int p0 = part * nkb / parts, p1 = (part + 1) * nkb / parts;
+  const int steps = (p1 - p0 + kStepKb - 1) / kStepKb;
+
+  // Inputs: the wave stages pairs kPairs w .. of a step; columns past the
+  // part and tokens past the batch read zeros.
+  const BufferResource x_res = MakeBuffer(x, unsigned(batch) * unsigned(ldx) * 4u);
+  float4 xv[kAhead][kPairs][2];
+  const auto load_x = [&](int step, float4 (&v)[kPairs][2]) {
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j) {
+      const int pair = wave * kPairs + j;
+      const int kb = p0 + step * kStepKb + pair / TT, token = tok0 + 16 * (pair % TT) + m;
+      const unsigned at = kb < p1 && token < batch
+                              ? (unsigned(token) * unsigned(ldx) + unsigned(kb * kTileCols + 8 * g)) * 4u
+                              : kOutOfRange;
+      v[j][0] = LoadF4(x_res, at);
+      v[j][1] = LoadF4(x_res, at + 16u);
+    }
+  };
+  const auto store_x = [&](uint4* stage, const float4 (&v)[kPairs][2]) {
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j) {
+      uint4 hi, mid, lo;
+      Operands(v[j][0], v[j][1], hi, mid, lo);
+      uint4* at = stage + (wave * kPairs + j) * 3 * 64 + lane;
+      at[0] = hi;
+      at[64] = mid;
+      at[128] = lo;
+    }
+  };
+  // Weights: the wave's column blocks in order (block i of it is column
+  // block p0 + kStepKb (i / kMine) + kg kMine + i % kMine); a buffer is
+  // loaded again as soon as its products are issued. Column blocks past the
+  // part read zeros, as their inputs do, so no step needs a branch.
+  // Tiles past the last one read the last one; their rows are never stored.
+  BufferResource w_res[RT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+    w_res[r] = MakeBuffer(tiles + std::size_t(min(tile0 + r, row_tiles - 1)) * nkb * (64 * NW),
+                          unsigned(nkb) * (1024u * NW));
+  const unsigned w_off = unsigned(lane) * 16u;
+  uint4 wv[kBufs][RT][NW];
+  const auto load_w = [&](int i, uint4 (&dst)[RT][NW]) {
+    const int kb = p0 + kStepKb * (i / kMine) + kg * kMine + i % kMine;
+    const unsigned off = kb < p1 ? w_off : kOutOfRange;
+    const unsigned at = kb < p1 ? unsigned(kb * NW) * 1024u : 0u;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int q = 0; q < NW; ++q)
+        dst[r][q] = LoadB128(w_res[r], off, at + unsigned(q) * 1024u);
+  };
+
+  // sum: the finished segments; acc: the open one; rest (formats in several
+  // parts): every product but hi times the weight's first part.
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 sum[RT][TT], acc[RT][TT], rest[NP > 1 ? RT : 1][NP > 1 ? TT : 1];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      sum[r][t] = acc[r][t] = zero;
+      if constexpr (NP > 1)
+        rest[r][t] = zero;
+    }
+
+  // One step's products. In one part: a pass of the mid and lo parts over the
+  // wave's column blocks, then one of the hi parts; each unit (a token group
+  // of a pass) reads the next unit's operands from LDS before its MFMAs, so
+  // that the matrix pipe does not wait for them, in a fixed order except at
+  // two K groups (a quarter of the step's time more there: 52 us against 46
+  // at 6144 x 2048, 512 rows; 27.8 against 29.3 at four groups, 256 rows).
+  const auto multiply = [&]<int kFirst>(const uint4* a, int next_block)
+                            __attribute__((always_inline)) {
+    if constexpr (NP == 1) {
+      constexpr int kUnits = 2 * kMine * TT;
+      const auto read = [&](int u, uint4 (&v)[2]) {
+        const uint4* at = a + u % (kMine * TT) * 3 * 64;
+        if (u < kMine * TT) {
+          v[0] = at[2 * 64];
+          v[1] = at[64];
+        } else {
+          v[0] = at[0];
+        }
+      };
+      constexpr bool kOrdered = KG != 2;
+      uint4 op[2][2];
+      if constexpr (kOrdered)
+        read(0, op[0]);
+      Unroll<kUnits>([&](auto unit) __attribute__((always_inline)) {
+        constexpr int u = unit, j = u / TT % kMine, t = u % TT;
+        constexpr bool small = u < kMine * TT;
+        if constexpr (kOrdered) {
+          if constexpr (u + 1 < kUnits)
+            read(u + 1, op[(u + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        } else {
+          read(u, op[u & 1]);
+        }
+#pragma unroll
+        for (int k = 0; k < (small ? 2 : 1); ++k)
+#pragma unroll
+          for (int r = 0; r < RT; ++r)
+            acc[r][t] = Mfma(op[u & 1][k], wv[kFirst + j][r][0], acc[r][t]);
+        if constexpr (!small && t == TT - 1)
+          load_w(next_block + j, wv[kFirst + j]);
+        if constexpr (kOrdered)
+          __builtin_amdgcn_sched_barrier(0);
+      });
+    } else {
+      Unroll<kMine>([&](auto block) __attribute__((always_inline)) {
+        constexpr int j = block;
+        uint4 av[TT][3];
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            av[t][k] = a[((j * TT + t) * 3 + k) * 64];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          uint4 wp[NP];
+          WeightParts<WF>(wv[kFirst + j][r], wp);
+#pragma unroll
+          for (int i = 0; i < NP; ++i)
+#pragma unroll
+            for (int k = 2; k >= 0; --k)
+#pragma unroll
+              for (int t = 0; t < TT; ++t)
+                if (i + k > 0)
+                  rest[r][t] = Mfma(av[t][k], wp[i], rest[r][t]);
+                else
+                  acc[r][t] = Mfma(av[t][k], wp[i], acc[r][t]);
+        }
+        load_w(next_block + j, wv[kFirst + j]);
+      });
+    }
+  };
+  const auto close_segment = [&]() {
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int t = 0; t < TT; ++t) {
+        sum[r][t] += acc[r][t];
+        acc[r][t] = zero;
+        asm volatile("" : "+v"(sum[r][t]), "+v"(acc[r][t]));
+      }
+  };
+
+  load_x(0, xv[0]);
+  if constexpr (kAhead == 2)
+    load_x(1, xv[1]);
+#pragma unroll
+  for (int i = 0; i < kBufs; ++i)
+    load_w(i, wv[i]);
+  store_x(s_mem, xv[0]);
+  // One step: the stage is visible and every wave is done with the other
+  // one; a later step's inputs load while this one multiplies (two steps
+  // ahead where a step is one column block a wave, shorter than the load).
+  const auto run_step = [&]<int kParity>(int step) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+    BlockBarrier();
+    // Past the last step every offset is out of range: nothing is read.
+    load_x(step + kAhead, xv[kAhead == 2 ? kParity : 0]);
+    const uint4* stage = s_mem + (step & 1) * kStage + kg * kMine * TT * 3 * 64 + lane;
+    multiply.template operator()<KG == 1 ? 0 : kParity * kMine>(stage, step * kMine + kBufs);
+    if ((step + 1) % KG == 0)
+      close_segment();
+    if (step + 1 < steps)
+      store_x(s_mem + ((step + 1) & 1) * kStage, xv[kAhead == 2 ? 1 - kParity : 0]);
+  };
+  int step = 0;
+  if constexpr (KG == 1) {
+    for (; step < steps; ++step)
+      run_step.template operator()<0>(step);
+  } else {
+    for (; step + 2 <= steps; step += 2) {
+      run_step.template operator()<0>(step);
+      run_step.template operator()<1>(step + 1);
+    }
+    if (step < steps)
+      run_step.template operator()<0>(step);
+  }
+  close_segment();
+  if constexpr (NP > 1)
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        sum[r][t] += rest[r][t];
+
+  // Lane l of a tile holds tokens 4 (l >> 4) + i, weight row l & 15.
+  float* yp = y + std::size_t(part) * part_stride;
+  constexpr int kOut = kSwiGLU ? RT / 2 : RT;  // output tiles a wave's rows give
+  const auto store = [&](int r, int t, const f32x4& a, const f32x4& b) {
+    const int row = ((kSwiGLU ? tile0 / 2 : tile0) + r) * 16 + m;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int token = tok0 + 16 * t + 4 * g + i;
+      if (row < out_rows && token < batch)
+        yp[std::size_t(token) * ldy + row] =
+            kSwiGLU ? (a[i] / (1.0f + expf(-a[i]))) * b[i] : a[i];
+    }
+  };
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int r = 0; r < kOut; ++r)
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+        store(r, t, sum[kSwiGLU ? 2 * r : r][t], sum[kSwiGLU ? 2 * r + 1 : r][t]);
+    return;
+  }
+  // The K groups' sums through LDS, added in group order; the groups share
+  // the output tiles.
+  f32x4* red = reinterpret_cast<f32x4*>(s_mem);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+      red[((kg * RG + rg) * RT + r) * (TT * 64) + t * 64 + lane] = sum[r][t];
+  __syncthreads();
+  const auto total = [&](int r, int t) {
+    f32x4 s = red[(rg * RT + r) * (TT * 64) + t * 64 + lane];
+#pragma unroll
+    for (int k = 1; k < KG; ++k)
+      s += red[((k * RG + rg) * RT + r) * (TT * 64) + t * 64 + lane];
+    return s;
+  };
+#pragma unroll
+  for (int u = 0; u < (kOut * TT + KG - 1) / KG; ++u) {
+    const int unit = u * KG + kg, r = unit / TT, t = unit % TT;
+    if (unit >= kOut * TT)
+      break;
+    const f32x4 a = total(kSwiGLU ? 2 * r : r, t);
+    store(r, t, a, kSwiGLU ? total(2 * r + 1, t) : a);
+  }
+}
+
 // Element (n, k) of a tile (row n < 16, column k < 32), in elements from
 // the tile's start.
 __host__ __device__ inline std::size_t TileIndex(int wf, int n, int k) {
@@ -272,11 +572,86 @@ void Launch(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, const
       int(ldy), int(out_rows), int(parts), std::size_t(batch) * ldy);
 }
 
+// The prompt rows' launch. RT row tiles a wave: 4 for BF16, 2 for the formats
+// whose weights split (their MFMAs per staged input are twice and three
+// times as many, and the parts take registers).
+template<int RT, int KG, int TT, bool kSwiGLU, int WF>
+void LaunchGemm(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, const float* x,
+                std::uint32_t ldx, std::uint32_t batch, float* y, std::uint32_t ldy,
+                std::uint32_t out_rows, std::uint32_t parts, hipStream_t stream) {
+  constexpr std::uint32_t kBlockTiles = RT * kWaves / KG;
+  const std::uint32_t row_blocks = (row_tiles + kBlockTiles - 1) / kBlockTiles;
+  const std::uint32_t token_blocks = (batch + 16 * TT - 1) / (16 * TT);
+  FloatGemmKernel<RT, KG, TT, kSwiGLU, WF><<<row_blocks * token_blocks * parts, kThreads, 0, stream>>>(
+      static_cast<const uint4*>(tiles), int(row_tiles), int(nkb), x, int(ldx), int(batch), y,
+      int(ldy), int(out_rows), int(row_blocks), int(token_blocks), int(parts),
+      std::size_t(batch) * ldy);
+}
+
+// Rows that take the prompt kernel: more than one token group, and inputs
+// that 32-bit buffer offsets reach.
+constexpr std::uint32_t kGemmMinRows = 17;
+bool PromptRows(std::uint32_t batch, std::uint32_t ldx) {
+  return batch >= kGemmMinRows && BufferFits(std::size_t(batch) * ldx * 4);
+}
+
+// Blocks of the prompt rows' kernel when a block owns `block_tiles` row tiles.
+std::uint32_t GemmBlocks(std::uint32_t row_tiles, std::uint32_t batch, std::uint32_t block_tiles) {
+  return (row_tiles + block_tiles - 1) / block_tiles * ((batch + 63) / 64);
+}
+
+// The block shape whose rounds on the 256 CUs cost least: `cost` is a round's
+// measured time at K = 2048, in microseconds (BF16, 64 tokens: 512 rows a
+// block 83, 256 rows 46, 128 rows 27.5, 64 rows 19.5). Blocks of 64 rows x 32
+// tokens where one round of them does (three fit a CU: 2048 x 2048 BF16 at
+// 64 rows 5.8 us against 8.6, F32 8.4 against 12.1; past one round the
+// weights' second read costs more, 7680 x 2048 at 96 rows 34.5 against 29.9)
+// and up to 32 tokens (the BF16 gate/up at 17 rows 12.0 us against 25).
+template<int WF, bool kSwiGLU>
+void GemmFormat(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, const float* x,
+                std::uint32_t ldx, std::uint32_t batch, float* y, std::uint32_t ldy,
+                std::uint32_t out_rows, std::uint32_t parts, hipStream_t s) {
+  const auto cost = [&](std::uint32_t block_tiles, double round) {
+    return double((GemmBlocks(row_tiles, batch, block_tiles) * parts + 255) / 256) * round;
+  };
+  const auto launch = [&](auto launcher) {
+    launcher(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, parts, s);
+  };
+  if (batch <= 32 || (row_tiles + 3) / 4 * ((batch + 31) / 32) * parts <= 256) {
+    launch(LaunchGemm<2, 4, 2, kSwiGLU, WF>);
+  } else if constexpr (WF == kBf16) {
+    const double c[4] = {cost(32, 83.0), cost(16, 46.0), cost(8, 27.5), cost(4, 19.5)};
+    const auto best = std::min_element(c, c + 4) - c;
+    if (best == 0)
+      launch(LaunchGemm<4, 1, 4, kSwiGLU, WF>);
+    else if (best == 1)
+      launch(LaunchGemm<4, 2, 4, kSwiGLU, WF>);
+    else if (best == 2)
+      launch(LaunchGemm<4, 4, 4, kSwiGLU, WF>);
+    else
+      launch(LaunchGemm<2, 4, 4, kSwiGLU, WF>);
+  } else {
+    const double c[3] = {cost(16, 80.0), cost(8, 46.0), cost(4, 28.0)};
+    const auto best = std::min_element(c, c + 3) - c;
+    if (best == 0)
+      launch(LaunchGemm<2, 1, 4, kSwiGLU, WF>);
+    else if (best == 1)
+      launch(LaunchGemm<2, 2, 4, kSwiGLU, WF>);
+    else
+      launch(LaunchGemm<2, 4, 4, kSwiGLU, WF>);
+  }
+}
+
 template<int WF>
 void LaunchFormat(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, const float* x,
                   std::uint32_t ldx, std::uint32_t batch, float* y, std::uint32_t ldy,
                   std::uint32_t out_rows, std::uint32_t parts, bool swiglu, hipStream_t s) {
-  if (swiglu) {
+  if (PromptRows(batch, ldx)) {
+    if (swiglu)
+      GemmFormat<WF, true>(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, 1, s);
+    else
+      GemmFormat<WF, false>(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, parts, s);
+  } else if (swiglu) {
     if (row_tiles >= 1024)
       Launch<4, true, WF>(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, 1, s);
     else
@@ -330,9 +705,12 @@ int lfm3_float_pack_host(uint32_t type, const void* src, uint32_t rows, uint32_t
 uint32_t lfm3_bf16_gemv_parts(uint32_t rows, uint32_t cols, uint32_t batch) {
   // Narrow outputs split K so that the grid reaches about 256 blocks; each
   // part keeps at least 16 column blocks (two a wave).
-  const std::uint32_t tiles = RowTilesOf(rows), groups = (batch + 15) / 16;
+  // Prompt rows count the blocks of 128 rows x 64 tokens.
+  const std::uint32_t tiles = RowTilesOf(rows);
   const std::uint32_t rt = tiles >= 1024 ? 4 : tiles >= 512 ? 2 : 1;
-  std::uint32_t blocks = (tiles + rt - 1) / rt * std::max(groups, 1u), parts = 1;
+  const std::uint32_t blocks =
+      batch >= kGemmMinRows ? GemmBlocks(tiles, batch, 8) : (tiles + rt - 1) / rt;
+  std::uint32_t parts = 1;
   while (parts < 8 && blocks * parts * 2 <= 256 && ColBlocks(cols) / (parts * 2) >= 16)
     parts *= 2;
   return parts;

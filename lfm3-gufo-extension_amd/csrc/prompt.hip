@@ -197,20 +197,6 @@ __device__ __forceinline__ void BufferToLds4(BufferResource res, unsigned lane_o
 }
 
 
-__device__ __forceinline__ void BlockBarrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Block b of a launch -> work item, XCD-major: blocks are dispatched to
-// the 8 XCDs round robin (b % 8), so XCD x gets the consecutive items
-// [first(x), first(x) + count(x)); items sharing weight rows are adjacent,
-// so their tiles come from HBM once per XCD and then from its L2.
-__device__ __forceinline__ int XcdMajorItem(int b, int blocks) {
-  const int q = blocks / 8, rem = blocks % 8, x = b % 8, i = b / 8;
-  return (x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + i;
-}
 
 // The SwiGLU GEMM's trailing blocks (lfm3_q8_gemm_swiglu_h16_rows): after
 // the GEMM blocks of a launch (blockIdx.x < gemm_blocks), each further

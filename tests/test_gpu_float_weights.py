@@ -227,3 +227,50 @@ def test_float_prompt_matches_oracle_steps(kind, n):
     g.close()
     gm.close()
     om.close()
+
+
+ALL_TYPES = dict(TYPES, bf16=L.TYPE_BF16)
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("M,K,B,parts", [
+    (1040, 160, 17, 1),    # the first batch past one token group; a part step at the end
+    (8192, 64, 769, 1),    # one K group a block (512 BF16 rows), 13 token blocks, one row in the last
+    (8192, 96, 385, 1),    # two K groups
+    (8176, 160, 193, 1),   # four K groups, a ragged last row block
+    (48, 2048, 65, 3),     # fewer rows than a block, K parts of unequal length
+    (37, 32, 64, 1),       # one column block: three K groups have none
+])
+def test_float_gemm_rows(kind, M, K, B, parts):
+    """The prompt rows' kernel against float64 and, per output, against the
+    same rows taken 16 at a time by the decode rows' kernel: both round only
+    their FP32 sums."""
+    tid = ALL_TYPES[kind]
+    h = synth(tid, f"fgr.{kind}.{M}x{K}", M, K)
+    m, w32 = FloatMatrix(tid, h, M, K), L.float_to_f32(h, tid).reshape(M, K)
+    x = (2.0 * L.normal(SEED, f"fgr.x.{M}x{K}.{B}", B * K)).reshape(B, K).astype(np.float32)
+    y = run(m, x, parts=parts)
+    check_fp64(y, w32, x)
+    scale = np.abs(x.astype(np.float64)) @ np.abs(w32.astype(np.float64)).T
+    for first in range(0, B, 16):
+        rows = run(m, np.ascontiguousarray(x[first:first + 16]))
+        assert np.all(np.abs(y[first:first + 16] - rows) <= 8e-6 * scale[first:first + 16] + 1e-30)
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("F,K,B", [(200, 96, 33), (7680, 64, 300), (3840, 96, 300)])
+def test_float_gemm_swiglu(kind, F, K, B):
+    """The SwiGLU epilogue over the prompt rows' kernel, in one and several
+    K groups, against float64: each product within 4e-6 of its absolute sum,
+    carried through y = silu(g) u (|silu'| <= 1.1, |silu(g)| <= |g|)."""
+    tid = ALL_TYPES[kind]
+    hg, hu = synth(tid, f"fgs.g.{kind}.{F}", F, K), synth(tid, f"fgs.u.{kind}.{F}", F, K)
+    m = FloatMatrix(tid, None, F, K, pairs=(hg, hu))
+    g32, u32 = (L.float_to_f32(h, tid).reshape(F, K) for h in (hg, hu))
+    x = L.normal(SEED, f"fgs.x.{F}.{B}", B * K).reshape(B, K).astype(np.float32)
+    y = run(m, x, swiglu=True)
+    x64, g64, u64 = (a.astype(np.float64) for a in (x, g32, u32))
+    g, u = x64 @ g64.T, x64 @ u64.T
+    eg, eu = (4e-6 * (np.abs(x64) @ np.abs(w).T) for w in (g64, u64))
+    bound = 1.1 * eg * (np.abs(u) + eu) + np.abs(g) * eu + 1e-6 * np.abs(g * u) + 1e-30
+    assert np.all(np.abs(y - g / (1 + np.exp(-g)) * u) <= bound)
