@@ -46,21 +46,48 @@ constexpr int kGemmRT = 4, kGemmTT = 4, kGemmStages = 3;
 // holds, decoded once at load into block 0's eight halves at byte 16 L and
 // block 1's at 1024 + 16 L), so the loop feeds them to the MFMA without the
 // per-chunk decode; the operands, and so every product, are the same.
-template<int WR, int WT, bool kHalf = false, int kStageCount = kGemmStages, int TT = kGemmTT>
+// KG > 1: the block's waves are KG groups of WR x WT, each with its own
+// stages and a KG-th of the block's chunks; the groups' sums meet in LDS
+// and add in group order.
+template<int WR, int WT, bool kHalf = false, int kStageCount = kGemmStages, int TT = kGemmTT,
+         int KG = 1>
 struct GemmShape {
-  static constexpr int kWR = WR, kWT = WT, kTT = TT;
+  static constexpr int kWR = WR, kWT = WT, kTT = TT, kKG = KG;
   static constexpr bool kHalfTiles = kHalf;
   static constexpr int kStages = kStageCount;  // LDS pipeline stages: 2 or 3
-  static constexpr int kWaves = WR * WT, kThreads = 64 * kWaves;
+  static constexpr int kWaves = WR * WT;       // waves of a K group
+  static constexpr int kThreads = 64 * kWaves * KG;
   static constexpr int kTiles = WR * kGemmRT;  // weight tiles a block
   static constexpr int kTokens = WT * TT * 16;
   static constexpr int kTileW = kHalf ? 2 * kTileCodeBytes : kTileCodeBytes;
   static constexpr int kW = kTokens * 128;
   static constexpr int kS = kW + kTiles * kTileW;
-  static constexpr int kBytes = kS + kTiles * kTileScales * 2;
+  static constexpr int kBytes = kS + kTiles * kTileScales * 2;  // a group's stage
+  static constexpr int kSums = (KG - 1) * kWaves * kGemmRT * TT * 64 * 16;
+  static_assert(kSums <= KG * kBytes, "the groups' sums fit the first stage array");
+  // Row maxima of 128 outputs come from the block that owns their 16 tiles.
+  static constexpr bool kMaxima = kTiles == 16 && KG == 1;
 };
 using WideShape = GemmShape<4, 2>;
 using NarrowShape = GemmShape<2, 2>;
+// Few rows leave most CUs idle under the 256- and 128-row blocks (77 rows:
+// gate/up 60 blocks, 44 us; 6144 x 2048 48 blocks, 24 us), and a block of
+// few tokens spends its steps waiting for memory: two chunks in flight and
+// 0.7-0.9 us a step whatever the shape. So these own 64 or 128 weight rows
+// and split their chunks over 2 to 4 K groups, which divides the steps and
+// multiplies the bytes in flight (75-150 KB of LDS, one block a CU).
+// Against the shapes they replace, alone, weights from HBM: 77 rows gate/up
+// 25.7 us (44.3), 6144 x 2048 12.3 (23.8), 2048 x 7680 in 4 parts 12.1
+// (22.9); 300 rows 6144 x 2048 19.4 (25.8); 2048 x 2048 at 200 rows in 2
+// parts 8.1 (13.7).
+template<bool kHalf>
+using Rows64Tokens32 = GemmShape<1, 2, kHalf, kGemmStages, 1, 4>;
+template<bool kHalf>
+using Rows64Tokens64 = GemmShape<1, 4, kHalf, kGemmStages, 1, 3>;
+template<bool kHalf>
+using Rows64Tokens128 = GemmShape<1, 4, kHalf, kGemmStages, 2, 2>;
+template<bool kHalf>
+using Rows128Tokens64 = GemmShape<2, 2, kHalf, kGemmStages, 2, 2>;
 // The same 256 x 128 block tile on FP16 tiles in 16 waves of 64 rows x 32
 // tokens: four waves a SIMD instead of two hide more of the LDS and MFMA
 // latency, for half again the LDS operand reads a MFMA (the SwiGLU GEMM
@@ -227,12 +254,13 @@ constexpr int kGemmSpinLimit = 1 << 20;
 // A trailing block of the SwiGLU GEMM: rows r0 .. r0 + kHiddenRows - 1 of
 // y (cols = the FFN width) once every GEMM block of their token block has
 // published. Loads read memory (sc1), where the GEMM blocks wrote.
-template<int T, int kTokens>
+template<class Shape>
 __device__ __forceinline__ void ConvertHidden(const HiddenHalves& t, const float* y, int ldy,
-                                              int cols, int n, const unsigned* row_max,
+                                              int cols, int n, unsigned* row_max,
                                               int row_blocks) {
+  constexpr int T = Shape::kThreads, kTokens = Shape::kTokens;
   static_assert(kTokens % kHiddenRows == 0, "a converter's rows lie in one token block");
-  constexpr int kHiddenLoads = kHiddenMaxCols / 4 / T;
+  constexpr int kHiddenLoads = (kHiddenMaxCols / 4 + T - 1) / T;
   __shared__ float s_rmax[kHiddenRows][T / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r0 = (int(blockIdx.x) - t.gemm_blocks) * kHiddenRows;
@@ -257,24 +285,19 @@ __device__ __forceinline__ void ConvertHidden(const HiddenHalves& t, const float
     }
   }
   __syncthreads();
-  // Each row's maximum over the partial maxima of the row blocks.
-  const BufferResource m_res = MakeBuffer(row_max, unsigned(row_blocks) * unsigned(n) * 4u);
-  float part[kHiddenRows];
+  float part[kHiddenRows] = {};
+  if constexpr (Shape::kMaxima) {
+    // Each row's maximum over the partial maxima of the row blocks.
+    const BufferResource m_res = MakeBuffer(row_max, unsigned(row_blocks) * unsigned(n) * 4u);
 #pragma unroll
-  for (int i = 0; i < kHiddenRows; ++i) {
-    const int r = r0 + i;
-    float m = 0.0f;
-    for (int b = tid; b < row_blocks; b += T)
-      m = fmaxf(m, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                       m_res, r < n ? unsigned(b * n + r) * 4u : kOutOfRange, 0,
-                       kCachePolicySc1)));
-    part[i] = WaveMax(m);
+    for (int i = 0; i < kHiddenRows; ++i) {
+      const int r = r0 + i;
+      for (int b = tid; b < row_blocks; b += T)
+        part[i] = fmaxf(part[i], __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                     m_res, r < n ? unsigned(b * n + r) * 4u : kOutOfRange, 0,
+                                     kCachePolicySc1)));
+    }
   }
-  if (lane == 0)
-#pragma unroll
-    for (int i = 0; i < kHiddenRows; ++i)
-      s_rmax[i][wave] = part[i];
-  __syncthreads();
   // Every row's values are loaded before the first conversion (at most
   // kHiddenLoads 16-byte loads a row and thread: cols <= kHiddenMaxCols), so
   // the block waits on memory once.
@@ -290,6 +313,33 @@ __device__ __forceinline__ void ConvertHidden(const HiddenHalves& t, const float
           y_res, r < n && v < cols / 4 ? unsigned(std::size_t(r) * ldy + 4 * v) * 4u : kOutOfRange,
           0, kCachePolicySc1);
     }
+  if constexpr (!Shape::kMaxima) {
+    // No block owned 128 outputs: 32 lanes hold those columns here, and
+    // their maximum is the partial one. (For the blocks that do own them the
+    // epilogue's maxima are the faster way: 512 rows 51.5 us against 52.3.)
+#pragma unroll
+    for (int i = 0; i < kHiddenRows; ++i)
+#pragma unroll
+      for (int j = 0; j < kHiddenLoads; ++j) {
+        float m =
+            fmaxf(fmaxf(fabsf(__uint_as_float(w[i][j].x)), fabsf(__uint_as_float(w[i][j].y))),
+                  fmaxf(fabsf(__uint_as_float(w[i][j].z)), fabsf(__uint_as_float(w[i][j].w))));
+#pragma unroll
+        for (int k = 16; k; k >>= 1)
+          m = fmaxf(m, __shfl_xor(m, k, 64));
+        const int v = tid + T * j;
+        if ((lane & 31) == 0 && r0 + i < n && v < cols / 4)
+          row_max[std::size_t(v / 32) * n + r0 + i] = __float_as_uint(m);
+        part[i] = fmaxf(part[i], m);
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < kHiddenRows; ++i) {
+    part[i] = WaveMax(part[i]);
+    if (lane == 0)
+      s_rmax[i][wave] = part[i];
+  }
+  __syncthreads();
   const int padded = (cols + kChunk - 1) / kChunk * kChunk;
 #pragma unroll
   for (int i = 0; i < kHiddenRows; ++i) {
@@ -335,25 +385,25 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
                              unsigned* __restrict__ row_max, const HiddenHalves tail) {
   constexpr int RT = kGemmRT, TT = Shape::kTT;
   using Stage = Shape;
-  constexpr int A_LOADS = Shape::kTokens * 8 / Shape::kThreads;  // 16-byte loads a lane
+  constexpr int KG = Shape::kKG, kGroupThreads = 64 * Shape::kWaves;
+  constexpr int A_LOADS = Shape::kTokens * 8 / kGroupThreads;  // 16-byte loads a lane
   constexpr int W_LOADS = Shape::kTiles / Shape::kWaves;         // tiles a wave loads
   constexpr int kTileW = Shape::kTileW;                           // bytes of a tile's chunk
   constexpr int W_PIECES = kTileW / kTileCodeBytes;               // 1 KB loads a tile
-  static_assert(A_LOADS * Shape::kThreads == Shape::kTokens * 8, "A loads cover the rows");
+  static_assert(A_LOADS * kGroupThreads == Shape::kTokens * 8, "A loads cover the rows");
   static_assert(W_LOADS * Shape::kWaves == Shape::kTiles, "W loads cover the tiles");
   static_assert(RT == 4 && Shape::kWR <= Shape::kWaves, "scale groups of four tiles");
   // One array per stage (not one indexed by stage) lets the compiler see
   // that a stage's reads never alias the other stages' loads in flight.
-  __shared__ __attribute__((aligned(16))) std::uint8_t s_st0[Stage::kBytes];
-  __shared__ __attribute__((aligned(16))) std::uint8_t s_st1[Stage::kBytes];
-  __shared__ __attribute__((aligned(16))) std::uint8_t s_st2[Shape::kStages == 3 ? Stage::kBytes : 16];
+  __shared__ __attribute__((aligned(16))) std::uint8_t s_st0[KG * Stage::kBytes];
+  __shared__ __attribute__((aligned(16))) std::uint8_t s_st1[KG * Stage::kBytes];
+  __shared__ __attribute__((aligned(16))) std::uint8_t s_st2[Shape::kStages == 3 ? KG * Stage::kBytes : 16];
   static_assert(Shape::kStages == 2 || Shape::kStages == 3, "two or three stage arrays");
 
   const bool publish = kSwiGLU && tail.out != nullptr;
   if constexpr (kSwiGLU) {
     if (publish && int(blockIdx.x) >= tail.gemm_blocks) {
-      ConvertHidden<Shape::kThreads, Shape::kTokens>(tail, y, ldy, rows_out, n, row_max,
-                                                     row_blocks);
+      ConvertHidden<Shape>(tail, y, ldy, rows_out, n, row_max, row_blocks);
       return;
     }
   }
@@ -361,12 +411,19 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
   const int tb = item % token_blocks, rb = (item / token_blocks) % row_blocks;
   const int part = item / (token_blocks * row_blocks);
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int block_wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = KG == 1 ? block_wave : block_wave % Shape::kWaves;
+  const int kg = KG == 1 ? 0 : block_wave / Shape::kWaves;
   const int wr = wave % Shape::kWR, wt = wave / Shape::kWR;
   const int btile0 = rb * Shape::kTiles;              // the block's first tile
   const int tile0 = btile0 + wr * RT;              // this wave's first tile
   const int tok0 = tb * Shape::kTokens;               // the block's first token
-  const int c_begin = part * nchunks / parts, c_end = (part + 1) * nchunks / parts;
+  // The group's chunks; every group takes the same number of steps.
+  const int p_begin = part * nchunks / parts, p_end = (part + 1) * nchunks / parts;
+  const int steps = (p_end - p_begin + KG - 1) / KG;
+  const int c_begin = p_begin + kg * steps;
+  const int c_end = KG == 1 ? p_end : min(p_end, c_begin + steps);
+  const int c_last = KG == 1 ? p_end : c_begin + steps;  // past c_end: no chunk
   y += std::size_t(part) * part_stride;
 
   // Sources as buffer resources (scalar registers), a scalar offset per
@@ -400,7 +457,8 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
       unsigned(min(btile0 + wave * 4 + (lane & 3), row_tiles - 1)) *
           unsigned(nchunks * kTileScales * 2) +
       unsigned((lane >> 2) * 4);
-  const auto issue = [&](int c, std::uint8_t* stage) {
+  const auto issue = [&](int c, std::uint8_t* stages) {
+    std::uint8_t* stage = stages + kg * Stage::kBytes;
 #pragma unroll
     for (int j = 0; j < A_LOADS; ++j)
       BufferToLds16(a_res, a_off[j], unsigned(c * kChunk * 2),
@@ -462,7 +520,8 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
     last[r] = zero;
     last_sc[r] = 0u;
   }
-  const auto compute = [&](const std::uint8_t* stage) {
+  const auto compute = [&](const std::uint8_t* stages) {
+    const std::uint8_t* stage = stages + kg * Stage::kBytes;
     uint4 q[RT];
     if constexpr (!Shape::kHalfTiles) {
 #pragma unroll
@@ -564,7 +623,8 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
   // flight), barrier (chunk c visible to every wave, and every wave done
   // with chunk c - 1), issue chunk c + 2 into chunk c - 1's stage, then
   // multiply chunk c. Loads get two chunks' compute to arrive.
-  issue(c_begin, s_st0);
+  if (KG == 1 || c_begin < c_end)
+    issue(c_begin, s_st0);
   if constexpr (Shape::kStages == 2) {
     // Two stages: step c waits for chunk c (the only loads in flight),
     // barrier (every wave done with chunk c - 1's stage), issues chunk
@@ -575,15 +635,16 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
       BlockBarrier();
       if (c + 1 < c_end)
         issue(c + 1, refill);
-      compute(stage);
+      if (KG == 1 || c < c_end)
+        compute(stage);
       __builtin_amdgcn_sched_barrier(0);
     };
     int c = c_begin;
-    for (; c + 2 <= c_end; c += 2) {
+    for (; c + 2 <= c_last; c += 2) {
       step2(c, s_st0, s_st1);
       step2(c + 1, s_st1, s_st0);
     }
-    if (c < c_end)
+    if (c < c_last)
       step2(c, s_st0, s_st1);
   } else {
   if (c_begin + 1 < c_end)
@@ -601,20 +662,21 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
     BlockBarrier();
     if (c + 2 < c_end)
       issue(c + 2, refill);
-    compute(stage);
+    if (KG == 1 || c < c_end)
+      compute(stage);
     __builtin_amdgcn_sched_barrier(0);
   };
   // Whole rounds of three chunks, then the ones left (no exits from inside
   // a round).
   int c = c_begin;
-  for (; c + 3 <= c_end; c += 3) {
+  for (; c + 3 <= c_last; c += 3) {
     step(c, s_st0, s_st2);
     step(c + 1, s_st1, s_st0);
     step(c + 2, s_st2, s_st1);
   }
-  if (c < c_end)
+  if (c < c_last)
     step(c, s_st0, s_st2);
-  if (c + 1 < c_end)
+  if (c + 1 < c_last)
     step(c + 1, s_st1, s_st0);
   }
 
@@ -624,6 +686,36 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       scale_fma(acc[r][TT - 1][i], last_sc[r], last[r][i], 1);
+
+  // The groups' sums: group 0 adds the others' to its own, in group order,
+  // and finishes the block.
+  if constexpr (KG > 1) {
+    f4* sums = reinterpret_cast<f4*>(s_st0) + wave * (RT * TT * 64) + lane;
+    constexpr int kGroup = Shape::kWaves * RT * TT * 64;
+    __syncthreads();
+    if (kg > 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+          sums[(kg - 1) * kGroup + (r * TT + t) * 64] =
+              f4{acc[r][t][0], acc[r][t][1], acc[r][t][2], acc[r][t][3]};
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+          for (int g = 0; g < KG - 1; ++g) {
+            const f4 other = sums[g * kGroup + (r * TT + t) * 64];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc[r][t][i] += other[i];
+          }
+    }
+  }
 
   // D layout: lane L holds tokens 16 t + 4 (L / 16) + i of weight row L % 16.
   const int sub = lane & 15, quad = lane >> 4;
@@ -646,63 +738,73 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
       token_off[t][i] = token < n ? unsigned(token) * unsigned(ldy) * 4u : kOutOfRange;
     }
   if constexpr (kSwiGLU) {
-    // Each token's max |y| over the block's rows (LDS), stored once per
-    // (row block, token) for the down projection's FP16 conversion.
-    __shared__ unsigned s_max[Shape::kTokens];
-    for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
-      s_max[i] = 0;
-    __syncthreads();
-    // Tiles (2 j, 2 j + 1) are a (gate, up) pair for output rows j * 16 + n.
-    unsigned row_off[RT / 2];
-#pragma unroll
-    for (int pr = 0; pr < RT / 2; ++pr) {
-      const int row = (tile0 / 2 + pr) * kTileRows + sub;
-      row_off[pr] = row < rows_out ? unsigned(row) * 4u : kOutOfRange;
+    // Each token's max |y| over the block's rows (LDS), stored once per (row
+    // block, token) for the down projection's FP16 conversion.
+    constexpr bool kMaxima = Shape::kMaxima;
+    __shared__ unsigned s_max[kMaxima ? Shape::kTokens : 1];
+    if constexpr (kMaxima) {
+      for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
+        s_max[i] = 0;
+      __syncthreads();
     }
+    if (kg == 0) {
+      // Tiles (2 j, 2 j + 1) are a (gate, up) pair for output rows j * 16 + n.
+      unsigned row_off[RT / 2];
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
+      for (int pr = 0; pr < RT / 2; ++pr) {
+        const int row = (tile0 / 2 + pr) * kTileRows + sub;
+        row_off[pr] = row < rows_out ? unsigned(row) * 4u : kOutOfRange;
+      }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float m = 0.0f;
+      for (int t = 0; t < TT; ++t) {
 #pragma unroll
-        for (int pr = 0; pr < RT / 2; ++pr) {
-          const float g = acc[2 * pr][t][i] * s[t][i], u = acc[2 * pr + 1][t][i] * s[t][i];
-          const float value = (g * (1.0f / (1.0f + expf(-g)))) * u;
-          const bool inside = token_off[t][i] != kOutOfRange && row_off[pr] != kOutOfRange;
-          const unsigned at = inside ? token_off[t][i] + row_off[pr] : kOutOfRange;
-          if (publish)  // uniform
-            StoreB32P<kCachePolicySc1>(y_res, at, __float_as_uint(value));
-          else
-            StoreF32(y_res, at, value);
-          m = inside ? fmaxf(m, fabsf(value)) : m;
+        for (int i = 0; i < 4; ++i) {
+          float m = 0.0f;
+#pragma unroll
+          for (int pr = 0; pr < RT / 2; ++pr) {
+            const float g = acc[2 * pr][t][i] * s[t][i], u = acc[2 * pr + 1][t][i] * s[t][i];
+            const float value = (g * (1.0f / (1.0f + expf(-g)))) * u;
+            const bool inside = token_off[t][i] != kOutOfRange && row_off[pr] != kOutOfRange;
+            const unsigned at = inside ? token_off[t][i] + row_off[pr] : kOutOfRange;
+            if (publish)  // uniform
+              StoreB32P<kCachePolicySc1>(y_res, at, __float_as_uint(value));
+            else
+              StoreF32(y_res, at, value);
+            m = inside ? fmaxf(m, fabsf(value)) : m;
+          }
+          if constexpr (kMaxima) {
+            m = fmaxf(m, __shfl_xor(m, 8, 64));
+            m = fmaxf(m, __shfl_xor(m, 4, 64));
+            m = fmaxf(m, __shfl_xor(m, 2, 64));
+            m = fmaxf(m, __shfl_xor(m, 1, 64));
+            if (sub == 0)
+              atomicMax(&s_max[wt * TT * 16 + t * 16 + 4 * quad + i], __float_as_uint(m));
+          }
         }
-        m = fmaxf(m, __shfl_xor(m, 8, 64));
-        m = fmaxf(m, __shfl_xor(m, 4, 64));
-        m = fmaxf(m, __shfl_xor(m, 2, 64));
-        m = fmaxf(m, __shfl_xor(m, 1, 64));
-        if (sub == 0)
-          atomicMax(&s_max[wt * TT * 16 + t * 16 + 4 * quad + i], __float_as_uint(m));
       }
     }
-    __syncthreads();
+    if constexpr (kMaxima)
+      __syncthreads();
     if (publish) {
       // The outputs and partial maxima through to memory, then the flag.
-      const BufferResource m_res =
-          MakeBuffer(row_max + std::size_t(rb) * n, unsigned(n) * 4u);
-      for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
-        StoreB32P<kCachePolicySc1>(m_res, tok0 + i < n ? unsigned(tok0 + i) * 4u : kOutOfRange,
-                                   s_max[i]);
+      if constexpr (kMaxima) {
+        const BufferResource m_res =
+            MakeBuffer(row_max + std::size_t(rb) * n, unsigned(n) * 4u);
+        for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
+          StoreB32P<kCachePolicySc1>(m_res, tok0 + i < n ? unsigned(tok0 + i) * 4u : kOutOfRange,
+                                     s_max[i]);
+      }
       __builtin_amdgcn_s_waitcnt(WaitVm(0));
       __syncthreads();
       if (tid == 0)
         __hip_atomic_store(tail.flags + tb * row_blocks + rb, tail.seq, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
-    } else if (row_max) {
+    } else if (kMaxima && row_max) {
       for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
         if (tok0 + i < n)
           row_max[std::size_t(rb) * n + tok0 + i] = s_max[i];
     }
-  } else {
+  } else if (kg == 0) {
     unsigned row_off[RT];
 #pragma unroll
     for (int r = 0; r < RT; ++r) {
@@ -753,34 +855,120 @@ __global__ void SumPartsKernel(float* __restrict__ y, std::size_t part_stride, i
   p[0] = sum;
 }
 
-// Blocks of one K part of a projection in the given shape.
+// The time of a launch in one of the block shapes, in microseconds: rounds
+// of the 256 CUs (one block a CU) times a round's start and end plus its
+// steps, and the traffic that grows with the blocks. Fitted to 70-100
+// launches of each shape on FP16 tiles, weights from HBM (2048 x 2048, 2048
+// x 7680, 3088 x 2048, 6144 x 2048, 20 to 512 rows, 1 to 8 parts), to within
+// 2.7 us each; the shape it picks is within 4% of the fastest on all but 12
+// of those 130 launches (where two blocks would share a CU, at most 25%).
+struct ShapeCost {
+  int tokens, tiles, groups;
+  float round, step, fill;
+};
 template<class Shape>
-int ShapeBlocks(int row_tiles, int tokens) {
-  return (row_tiles + Shape::kTiles - 1) / Shape::kTiles *
-         ((tokens + Shape::kTokens - 1) / Shape::kTokens);
+constexpr ShapeCost CostOf(float round, float step, float fill) {
+  return {Shape::kTokens, Shape::kTiles, Shape::kKG, round, step, fill};
+}
+constexpr ShapeCost kShapeCosts[] = {
+    CostOf<Rows64Tokens32<true>>(1.55f, 0.758f, 0.083f),
+    CostOf<Rows64Tokens64<true>>(1.91f, 0.680f, 0.215f),
+    CostOf<Rows64Tokens128<true>>(3.11f, 0.648f, 0.224f),
+    CostOf<Rows128Tokens64<true>>(3.22f, 0.708f, 0.234f),
+    CostOf<NarrowHalfShape>(3.28f, 0.558f, 0.232f),
+    CostOf<WideHalfShape>(5.52f, 0.872f, 0.435f),
+};
+constexpr int kShapes = sizeof(kShapeCosts) / sizeof(kShapeCosts[0]);
+constexpr int kWide = kShapes - 1;
+
+int ShapeBlocks(const ShapeCost& s, int row_tiles, int tokens) {
+  return (row_tiles + s.tiles - 1) / s.tiles * ((tokens + s.tokens - 1) / s.tokens);
 }
 
-// The block shape of a projection: wide when its blocks alone fill most of
-// the 256 CUs, narrow (two blocks a CU) otherwise.
-bool NarrowGemm(int row_tiles, int tokens) {
-  return ShapeBlocks<WideShape>(row_tiles, tokens) < 192;
+float LaunchCost(const ShapeCost& s, int row_tiles, int tokens, int nchunks, int parts) {
+  const int blocks = ShapeBlocks(s, row_tiles, tokens) * parts;
+  const int steps = (nchunks + parts * s.groups - 1) / (parts * s.groups);
+  return float((blocks + 255) / 256) * (s.round + s.step * float(steps)) +
+         s.fill * float(steps) * float(blocks) / 256.0f;
 }
 
-// K parts for a prompt GEMM: double while the blocks stay within 320
-// (wide shape: one round on the 256 CUs with a quarter over) or 384
-// (narrow shape) and each part keeps at least 4 chunks, at most 8 parts.
-// Each part costs its consumer one more FP32 output pass; on the model's
-// 512-token projections these limits give the fastest GEMM plus part
-// reads (2048 x 2048: 4 parts; 6144 x 2048: 2; 2048 x 7680: 4).
+// Flags of a SwiGLU launch with trailing conversion blocks: one per GEMM
+// block. The count grows with the tokens, so a buffer made for some tokens
+// serves every call of fewer; a shape that needs more is not taken.
+std::size_t SwiGLUFlags(int row_tiles, std::uint32_t tokens) {
+  const ShapeCost& wide = kShapeCosts[kWide];
+  return std::size_t(row_tiles + wide.tiles - 1) / wide.tiles *
+         std::max<std::size_t>(4, (std::size_t(tokens) + wide.tokens - 1) / wide.tokens);
+}
+
+// The shape of least cost. The code and FP16 tiles of a matrix take the same
+// one: K groups change the order of a sum.
+int BestShape(int row_tiles, int tokens, int nchunks, int parts, bool swiglu) {
+  int best = kWide;
+  float least = LaunchCost(kShapeCosts[kWide], row_tiles, tokens, nchunks, parts);
+  for (int i = 0; i < kWide; ++i) {
+    const float cost = LaunchCost(kShapeCosts[i], row_tiles, tokens, nchunks, parts);
+    if (cost < least && (!swiglu || std::size_t(ShapeBlocks(kShapeCosts[i], row_tiles, tokens)) <=
+                                        SwiGLUFlags(row_tiles, std::uint32_t(tokens)))) {
+      best = i;
+      least = cost;
+    }
+  }
+  return best;
+}
+
+// K parts for a prompt GEMM: the count, among 1, 2, 4 and 8 parts of at
+// least 4 chunks, whose launch and parts cost least. Parts cost their
+// consumer: 1 us between a residual norm or heads kernel that adds them
+// (under 1 us for the first) and one that needs lfm3_sum_parts (4 us a
+// launch), and an FP32 output pass for each further one (512 rows of 2048:
+// the norm takes 7.3 us with 4 parts, 8.8 with 8). 2048 x 2048: 4 parts at
+// 20 rows (5.1 us; 8.1 in one), 2 at 77 (6.0; 8.2 in one, 5.7 in 8) and at
+// 512 (11.1; 11.9 in 4); 2048 x 7680: 4 at 512 rows (28.5; 27.0 in 8); 3088
+// x 2048: one from 77 rows on. Under 16 chunks (K below 1024, which no
+// fitted launch had) a launch is mostly its start and end: parts double
+// while blocks of 128 x 128 stay within 384.
 int PromptParts(int row_tiles, int tokens, int nchunks) {
-  const bool narrow = NarrowGemm(row_tiles, tokens);
-  const int blocks = narrow ? ShapeBlocks<NarrowShape>(row_tiles, tokens)
-                            : ShapeBlocks<WideShape>(row_tiles, tokens);
-  const int limit = narrow ? 384 : 320;
-  int parts = 1;
-  while (parts < 8 && blocks * parts * 2 <= limit && nchunks / (parts * 2) >= 4)
-    parts *= 2;
-  return parts;
+  if (nchunks < 16) {
+    const int blocks = (row_tiles + 7) / 8 * ((tokens + 127) / 128);
+    int parts = 1;
+    while (parts < 8 && blocks * parts * 2 <= 384 && nchunks / (parts * 2) >= 4)
+      parts *= 2;
+    return parts;
+  }
+  int best = 1;
+  float least = 0.0f;
+  for (int parts = 1; parts <= 8 && (parts == 1 || nchunks / parts >= 4); parts *= 2) {
+    const int shape = BestShape(row_tiles, tokens, nchunks, parts, false);
+    const float cost = LaunchCost(kShapeCosts[shape], row_tiles, tokens, nchunks, parts) +
+                       (parts > 1 ? 1.0f : 0.0f) +
+                       float(parts - 1) * (0.1f + 7e-6f * float(tokens) * float(row_tiles));
+    if (parts == 1 || cost < least) {
+      best = parts;
+      least = cost;
+    }
+  }
+  return best;
+}
+
+// Each token's max |y| over 128 output columns (blockIdx.x), for the SwiGLU
+// launches whose blocks own fewer (the trailing blocks find them
+// themselves): 32 lanes a token.
+__global__ void RowMaximaKernel(const float* __restrict__ y, int ldy, int cols, int n,
+                                unsigned* __restrict__ row_max) {
+  const int token = blockIdx.y * 8 + int(threadIdx.x >> 5), lane = threadIdx.x & 31;
+  float m = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int col = blockIdx.x * 128 + 32 * j + lane;
+    if (token < n && col < cols)
+      m = fmaxf(m, fabsf(y[std::size_t(token) * ldy + col]));
+  }
+#pragma unroll
+  for (int k = 16; k; k >>= 1)
+    m = fmaxf(m, __shfl_xor(m, k, 64));
+  if (token < n && lane == 0)
+    row_max[std::size_t(blockIdx.x) * n + token] = __float_as_uint(m);
 }
 
 // The kernel addresses codes, scales, activations and each output part
@@ -809,6 +997,23 @@ void LaunchGemm(const void* codes, const void* scales, int row_tiles, int nchunk
       static_cast<const std::uint8_t*>(codes), static_cast<const Half*>(scales), row_tiles,
       nchunks, reinterpret_cast<const Half*>(a), int(lda), a_scale, int(tokens), y, int(ldy),
       int(rows), row_blocks, token_blocks, parts, part_stride, row_max, tail);
+  if constexpr (kSwiGLU && !Shape::kMaxima)
+    if (row_max && !tail.out)
+      RowMaximaKernel<<<dim3((rows + 127) / 128, (tokens + 7) / 8), 256, 0, stream>>>(
+          y, int(ldy), int(rows), int(tokens), row_max);
+}
+
+// The launcher of shape `i` (kShapeCosts) on FP16 or code tiles.
+template<bool kSwiGLU>
+auto Launcher(int i, bool half) {
+  constexpr decltype(&LaunchGemm<kSwiGLU, WideShape>) kLaunchers[2][kShapes] = {
+      {LaunchGemm<kSwiGLU, Rows64Tokens32<false>>, LaunchGemm<kSwiGLU, Rows64Tokens64<false>>,
+       LaunchGemm<kSwiGLU, Rows64Tokens128<false>>, LaunchGemm<kSwiGLU, Rows128Tokens64<false>>,
+       LaunchGemm<kSwiGLU, NarrowShape>, LaunchGemm<kSwiGLU, WideShape>},
+      {LaunchGemm<kSwiGLU, Rows64Tokens32<true>>, LaunchGemm<kSwiGLU, Rows64Tokens64<true>>,
+       LaunchGemm<kSwiGLU, Rows64Tokens128<true>>, LaunchGemm<kSwiGLU, Rows128Tokens64<true>>,
+       LaunchGemm<kSwiGLU, NarrowHalfShape>, LaunchGemm<kSwiGLU, WideHalfShape>}};
+  return kLaunchers[half][i];
 }
 
 }  // namespace
@@ -844,7 +1049,7 @@ int lfm3_half_rows(const float* x, std::uint32_t ldx, const unsigned* row_max,
 }
 
 std::uint32_t lfm3_q8_gemm_swiglu_max_blocks(std::uint32_t rows) {
-  return (2 * RowTiles(rows) + WideShape::kTiles - 1) / WideShape::kTiles;
+  return (rows + 127) / 128;
 }
 
 std::uint32_t lfm3_q8_gemm_parts(std::uint32_t rows, std::uint32_t cols,
@@ -884,11 +1089,8 @@ int Gemm(const void* tiles, bool half, const void* scales, std::uint32_t rows,
       (reinterpret_cast<std::uintptr_t>(a) & 15) ||
       !GemmOperandsFit(RowTiles(rows), Chunks(cols), tokens, lda, ldy, half))
     return Fail(LFM3_E_INVALID, "unsupported LFM3 Q8_0 prompt GEMM shape");
-  const bool narrow = NarrowGemm(int(RowTiles(rows)), int(tokens));
-  const auto launch = half ? (narrow ? LaunchGemm<false, NarrowHalfShape>
-                                     : LaunchGemm<false, WideHalfShape>)
-                           : (narrow ? LaunchGemm<false, NarrowShape>
-                                     : LaunchGemm<false, WideShape>);
+  const auto launch = Launcher<false>(
+      BestShape(int(RowTiles(rows)), int(tokens), int(Chunks(cols)), int(parts), false), half);
   launch(tiles, scales, int(RowTiles(rows)), int(Chunks(cols)), a, lda, a_scale, tokens, y, ldy,
          rows, int(parts), std::size_t(ldy) * tokens, nullptr, static_cast<hipStream_t>(stream),
          HiddenHalves{});
@@ -904,18 +1106,11 @@ int GemmSwiGLU(const void* tiles, bool half, const void* scales, std::uint32_t r
       ldy < rows || (reinterpret_cast<std::uintptr_t>(a) & 15) ||
       !GemmOperandsFit(2 * RowTiles(rows), Chunks(cols), tokens, lda, ldy, half))
     return Fail(LFM3_E_INVALID, "unsupported LFM3 Q8_0 prompt SwiGLU shape");
-  const auto launch = half ? LaunchGemm<true, WideHalfShape> : LaunchGemm<true, WideShape>;
+  const auto launch = Launcher<true>(
+      BestShape(int(2 * RowTiles(rows)), int(tokens), int(Chunks(cols)), 1, true), half);
   launch(tiles, scales, int(2 * RowTiles(rows)), int(Chunks(cols)), a, lda, a_scale, tokens, y,
          ldy, rows, 1, 0, row_max, static_cast<hipStream_t>(stream), tail);
   return HipStatus(hipGetLastError(), "LFM3 Q8_0 prompt SwiGLU launch");
-}
-
-// Flags of a SwiGLU launch with trailing conversion blocks: one per GEMM block.
-std::size_t SwiGLUFlags(std::uint32_t rows, std::uint32_t tokens) {
-  const std::size_t row_blocks = (2 * RowTiles(rows) + WideHalfShape::kTiles - 1) /
-                                 WideHalfShape::kTiles;
-  const std::size_t token_blocks = (tokens + WideHalfShape::kTokens - 1) / WideHalfShape::kTokens;
-  return row_blocks * token_blocks;
 }
 
 }  // namespace
@@ -930,7 +1125,7 @@ int lfm3_q8_gemm(const void* codes, const void* scales, std::uint32_t rows,
 }
 
 std::size_t lfm3_q8_gemm_swiglu_flags_bytes(std::uint32_t rows, std::uint32_t tokens) {
-  return rows && tokens ? SwiGLUFlags(rows, tokens) * sizeof(unsigned) : 0;
+  return rows && tokens ? SwiGLUFlags(int(2 * RowTiles(rows)), tokens) * sizeof(unsigned) : 0;
 }
 
 int lfm3_q8_gemm_swiglu_h16_rows(const void* halves, const void* scales, std::uint32_t rows,

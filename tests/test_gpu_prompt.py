@@ -180,6 +180,54 @@ def test_gemm_half_tiles_identical(M, K, n, parts, swiglu):
     assert ok, err
 
 
+@pytest.mark.parametrize("M,K,n,parts", [
+    (2050, 64, 16, 1),     # 64 x 32 blocks, one chunk for four K groups; a ragged last block
+    (2050, 1088, 33, 2),   # two token blocks of 32 or one of 64; 17 chunks in two parts
+    (6144, 448, 64, 1),    # 64 x 64 blocks: seven chunks over three K groups
+    (6144, 448, 65, 2),    # 64 x 128 blocks, the second half nearly empty
+    (6144, 2048, 300, 1),  # 128 x 64 blocks
+    (6144, 2048, 385, 1),  # 128 x 128 blocks, one row in the last
+    (16, 7680, 17, 8),     # one weight tile
+])
+def test_gemm_block_shapes(M, K, n, parts):
+    """Row counts and K lengths at the edges of the block shapes: FP16 and
+    code tiles bit-exact, each within the gate of FP64, and nothing depends
+    on the rows beside a row (its outputs alone, 16 rows at a time, differ
+    only by the order of the K groups' sums)."""
+    g = L.q8(SEED, f"bs.{M}.{K}", M, K)
+    m = DeviceMatrix(g, M, K)
+    x = L.normal(SEED, f"bs.x.{M}.{K}.{n}", n * K).reshape(n, K)
+    a, b = gemm(m, x, parts, half=True), gemm(m, x, parts)
+    assert np.array_equal(a, b)
+    inputs, _ = O.half_rows(x)
+    want = inputs.astype(np.float64) @ L.q8_dequant(g, M, K).T
+    ok, err = within(a, want)
+    assert ok, err
+    first = gemm(m, np.ascontiguousarray(x[:16]), parts, half=True)
+    ok, err = within(a[:16], first.astype(np.float64))
+    assert ok, err
+
+
+@pytest.mark.parametrize("F,K,n", [(208, 128, 16), (7680, 64, 77), (7680, 128, 129),
+                                   (208, 192, 300)])
+def test_gemm_swiglu_block_shapes(F, K, n):
+    """SwiGLU in the blocks of few rows: within the gate of FP64, and the
+    partial maxima of every 128 outputs exact though no block owns them."""
+    g, u = L.q8(SEED, f"bw.g{F}", F, K), L.q8(SEED, f"bw.u{F}", F, K)
+    m = DeviceMatrix(g, F, K, interleave_with=u)
+    x = L.normal(SEED, f"bw.x{F}.{n}", n * K).reshape(n, K)
+    y, rm = gemm(m, x, swiglu=True, half=True)
+    inputs, _ = O.half_rows(x)
+    gv = inputs.astype(np.float64) @ L.q8_dequant(g, F, K).T
+    uv = inputs.astype(np.float64) @ L.q8_dequant(u, F, K).T
+    ok, err = within(y, gv / (1 + np.exp(-gv)) * uv)
+    assert ok, err
+    maxima = rm.view(np.float32)
+    assert maxima.shape[0] == -(-F // 128)
+    for b in range(maxima.shape[0]):
+        assert np.array_equal(maxima[b], np.abs(y[:, 128 * b:128 * (b + 1)]).max(axis=1))
+
+
 @pytest.mark.parametrize("F,K,ns", [(7680, 2048, (512, 300)), (192, 128, (20, 133)),
                                     (7680, 2048, (16, 512))])
 def test_gemm_swiglu_rows_is_gemm_then_half_rows(F, K, ns):
