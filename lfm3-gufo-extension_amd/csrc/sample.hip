@@ -22,11 +22,12 @@
 // Two launches. The first splits every row into slices of 4096 logits, one
 // block each, so a batch of 8 rows of 128000 fills 256 CUs: the slice is
 // read from HBM once into LDS (penalized there) and reduced to its best
-// greedy key, its (max, weight sum), or its own top-k candidates in index
-// order (keys above its k-th, then its lowest-index ties). The global top-k
-// is among the slices' candidates, in global index order wherever keys tie.
-// The second launch, one block per row, selects the k-th key among the
-// candidates by radix select, sorts the k winners in LDS and picks; for
+// greedy key, its (max, weight sum), or its own top-k candidates (sorted, or
+// keys above its k-th in index order, then its lowest-index ties). The global
+// top-k is among the slices' candidates, in global index order wherever keys
+// tie. The second launch, one block per row, takes the k winners among the
+// candidates (ranked behind a bound, or by radix select and a sort) and
+// picks; for
 // the whole vocabulary it finds the slice that holds the target from the
 // slices' sums and walks that slice's weights in index order.
 #include <cmath>
@@ -198,6 +199,61 @@ __device__ float BlockSum(float v, float* s_f) {
   return b;
 }
 
+// The top-k of few: a lower bound of the k-th largest key from a sample of
+// the keys, the keys at or above the bound in index order, and each one's
+// rank among them by counting. A radix select of the same keys is four
+// passes of LDS atomics that collide on the few exponents logits have:
+// top-k 50 of 8 x 128000 took 24.9 us with it in both launches and takes
+// 17.9 here (k = 120, 4 rows: 40.3 and 23.3; k = 5: 22.0 and 13.8). What is
+// left is the two launches' latency: a slice's loads, its scan, the
+// candidates' round trip. Past kBoundMaxK the sample is too small to cut the
+// keys down, and more than kBoundMaxKeys at or above the bound (many equal
+// logits) are left to the radix select.
+constexpr int kBoundMaxK = 128, kBoundMaxKeys = 512;
+
+// The largest multiple t of 2^14 with at least k of the wave's keys (R a
+// lane, zeros for none) at or above it: every lane's result. 18 bits keep
+// the exponent and 9 bits of the value, well inside the gap between the
+// bound and the k-th key that a sample leaves anyway.
+template<int R>
+__device__ __forceinline__ unsigned KeyBound(const unsigned (&key)[R], int k) {
+  unsigned t = 0;
+  for (int bit = 31; bit >= 14; --bit) {
+    const unsigned next = t | (1u << bit);
+    int at_least = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      at_least += __popcll(__ballot(key[r] >= next));
+    t = at_least >= k ? next : t;
+  }
+  return t;
+}
+
+// Rank of key j of n in LDS: keys above it, then equal keys before it. Read
+// four at a time; the entries up to the next multiple of 16 are zero.
+__device__ __forceinline__ int RankOf(const unsigned* s_key, int n, int j) {
+  const unsigned mine = s_key[j];
+  int rank = 0;
+  for (int q0 = 0; q0 < n; q0 += 16) {
+    uint4 k4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      k4[i] = *reinterpret_cast<const uint4*>(&s_key[q0 + 4 * i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned other[4] = {k4[i].x, k4[i].y, k4[i].z, k4[i].w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        rank += other[c] > mine || (other[c] == mine && q0 + 4 * i + c < j) ? 1 : 0;
+    }
+  }
+  return rank;
+}
+
+__device__ __forceinline__ float OrderedValue(unsigned key) {
+  return __uint_as_float((key & 0x80000000u) ? key ^ 0x80000000u : ~key);
+}
+
 struct SliceArgs {
   const float* logits;
   int ld;
@@ -224,6 +280,13 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
   const int begin = slice * kSliceLen, len = min(kSliceLen, a.cols - begin);
   const float* x = (a.row_ptrs ? a.row_ptrs[row] : a.logits + std::size_t(row) * a.ld) + begin;
   const bool penalize = a.penalty_ids && a.n_penalty > 0 && a.penalty != 1.0f;
+  // Every load of the slice first (zeros past its end), the penalty's bits
+  // while they are in flight.
+  const BufferResource x_res = MakeBuffer(x, unsigned(len) * 4u);
+  float raw[kSliceLen / kSliceThreads];
+#pragma unroll
+  for (int q = 0; q < kSliceLen / kSliceThreads; ++q)
+    raw[q] = __uint_as_float(LoadB32(x_res, unsigned(tid + kSliceThreads * q) * 4u));
   if (penalize) {
     for (int i = tid; i < kSliceLen / 32; i += kSliceThreads)
       s_bits[i] = 0u;
@@ -236,8 +299,11 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
     }
     __syncthreads();
   }
-  for (int i = tid; i < len; i += kSliceThreads) {
-    float l = x[i];
+  constexpr int kOwn = kSliceLen / kSliceThreads;
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    const int i = tid + kSliceThreads * q;
+    float l = raw[q];
     if (penalize && (s_bits[i >> 5] >> (i & 31) & 1u))
       l = Penalized(l, a.penalty);
     s_v[i] = l;
@@ -283,14 +349,7 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
     }
     return;
   }
-  unsigned kth, ties;
-  SelectKth<kSliceThreads>(len, unsigned(k), [&](int i) { return OrderedBits(s_v[i]); },
-                           s_hist, s_sel, kth, ties);
-  // Thread t owns the kOwn consecutive elements from kOwn t: it counts its
-  // keys above the k-th and equal to it, one block scan of the packed
-  // counts gives its output offsets, and it writes its winners in index
-  // order (the lowest-index ties first).
-  constexpr int kOwn = kSliceLen / kSliceThreads;
+  // Thread t owns the kOwn consecutive elements from kOwn t.
   float vals[kOwn];
 #pragma unroll
   for (int q = 0; q < kOwn / 4; ++q) {
@@ -300,6 +359,57 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
     vals[4 * q + 2] = f.z;
     vals[4 * q + 3] = f.w;
   }
+  if (k <= kBoundMaxK) {
+    // The bound from the threads' largest keys; the winners go out by rank,
+    // so in descending order, the lower index first where keys tie.
+    __shared__ __attribute__((aligned(16))) unsigned s_best[kSliceThreads];
+    __shared__ __attribute__((aligned(16))) unsigned s_cand[kBoundMaxKeys + 16];
+    __shared__ unsigned s_at[kBoundMaxKeys];
+    unsigned best = 0u;
+#pragma unroll
+    for (int j = 0; j < kOwn; ++j)
+      best = tid * kOwn + j < len ? max(best, OrderedBits(vals[j])) : best;
+    s_best[tid] = best;
+    __syncthreads();
+    const uint4 b4 = *reinterpret_cast<const uint4*>(&s_best[4 * (tid & 63)]);
+    const unsigned b[4] = {b4.x, b4.y, b4.z, b4.w};
+    const unsigned bound = KeyBound(b, k);
+    unsigned own = 0;
+#pragma unroll
+    for (int j = 0; j < kOwn; ++j)
+      own += tid * kOwn + j < len && OrderedBits(vals[j]) >= bound ? 1u : 0u;
+    unsigned found;
+    unsigned at = BlockScan<kSliceThreads>(own, s_wave, &found);
+    if (found <= unsigned(kBoundMaxKeys)) {  // uniform
+      if (tid < 16)
+        s_cand[found + tid] = 0u;
+#pragma unroll
+      for (int j = 0; j < kOwn; ++j) {
+        const int i = tid * kOwn + j;
+        const unsigned key = OrderedBits(vals[j]);
+        if (i < len && key >= bound) {
+          s_cand[at] = key;
+          s_at[at] = unsigned(begin + i);
+          ++at;
+        }
+      }
+      __syncthreads();
+      for (int j = tid; j < int(found); j += kSliceThreads) {
+        const int rank = RankOf(s_cand, int(found), j);
+        if (rank < k) {
+          out_v[rank] = OrderedValue(s_cand[j]);
+          out_i[rank] = s_at[j];
+        }
+      }
+      return;
+    }
+  }
+  unsigned kth, ties;
+  SelectKth<kSliceThreads>(len, unsigned(k), [&](int i) { return OrderedBits(s_v[i]); },
+                           s_hist, s_sel, kth, ties);
+  // It counts its keys above the k-th and equal to it, one block scan of the
+  // packed counts gives its output offsets, and it writes its winners in
+  // index order (the lowest-index ties first).
   unsigned counts = 0;
 #pragma unroll
   for (int j = 0; j < kOwn; ++j) {
@@ -380,18 +490,25 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
       s_z[s] = stats[4 * s + 1];
     }
     __syncthreads();
+    float top_m = -INFINITY;
+#pragma unroll 8
+    for (int s = 0; s < a.slices; ++s)
+      top_m = fmaxf(top_m, s_m[s]);
+    __syncthreads();
+    for (int s = tid; s < a.slices; s += kPickThreads)
+      s_z[s] *= expf((s_m[s] - top_m) * a.inv_t);
+    __syncthreads();
     if (tid == 0) {
-      float top = -INFINITY;
-      for (int s = 0; s < a.slices; ++s)
-        top = fmaxf(top, s_m[s]);
+      const float top = top_m;
       float total = 0.0f;
+#pragma unroll 8
       for (int s = 0; s < a.slices; ++s)
-        total += s_z[s] * expf((s_m[s] - top) * a.inv_t);
+        total += s_z[s];
       const float target = u * total;
       float run = 0.0f;
       int pick = -1, last = 0;
       for (int s = 0; s < a.slices; ++s) {
-        const float z = s_z[s] * expf((s_m[s] - top) * a.inv_t);
+        const float z = s_z[s];
         if (z > 0.0f)
           last = s;
         if (pick < 0 && run + z > target) {
@@ -452,15 +569,27 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
     float before = incl - own;
     for (int v = 0; v < wave; ++v)
       before += s_f[v];
+    // The last element with weight and the first past the target: of the
+    // thread, then of the wave, then one LDS atomic a wave (one an element
+    // was 4096 of them on one address).
     float run = before;
+    int own_last = -1, own_pick = 0x7fffffff;
     for (int j = 0; j < 4; ++j) {
       const int i = 4 * tid + j;
       if (w[j] > 0.0f) {
-        atomicMax(&s_last, i);
+        own_last = i;
         if (run + w[j] > target)
-          atomicMin(&s_pick, i);
+          own_pick = min(own_pick, i);
       }
       run += w[j];
+    }
+    for (int off = 1; off < 64; off <<= 1) {
+      own_last = max(own_last, __shfl_xor(own_last, off, 64));
+      own_pick = min(own_pick, __shfl_xor(own_pick, off, 64));
+    }
+    if (lane == 0) {
+      atomicMax(&s_last, own_last);
+      atomicMin(&s_pick, own_pick);
     }
     __syncthreads();
     if (tid == 0) {
@@ -479,102 +608,151 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   // The candidates' keys are read from the workspace once into LDS when
   // they fit, so the select's passes and the compaction read LDS.
   constexpr int kStagedKeys = 8192;
-  __shared__ unsigned s_cand[kStagedKeys];
+  __shared__ unsigned s_cand[kStagedKeys], s_ci[kStagedKeys];
   const bool staged = n <= kStagedKeys;
   if (staged) {
-    for (int i = tid; i < n; i += kPickThreads)
+#pragma unroll 4
+    for (int i = tid; i < n; i += kPickThreads) {
       s_cand[i] = OrderedBits(cv[i]);
+      s_ci[i] = ci[i];
+    }
     __syncthreads();
   }
   const auto key_of = [&](int i) { return staged ? s_cand[i] : OrderedBits(cv[i]); };
-  unsigned kth, ties;
-  SelectKth<kPickThreads>(n, unsigned(k), key_of, s_hist, s_sel, kth, ties);
   // Thread t owns `per` consecutive candidates (the slices' candidates in
-  // slice order, so in global index order where keys tie): counts, one
-  // block scan, then the winners in order.
+  // slice order, so in global index order where keys tie).
   const int per = (n + kPickThreads - 1) / kPickThreads, i0 = tid * per;
-  unsigned counts = 0;
-  for (int j = 0; j < per; ++j) {
-    const int i = i0 + j;
-    if (i < n) {
-      const unsigned key = key_of(i);
-      counts += key > kth ? (1u << kUpShift) : key == kth ? 1u : 0u;
+  // The bound from each slice's first candidates (its largest, where it
+  // ranked them), at least 2 k of them in all where there are as many. A
+  // bound above +0 keeps out the padding and both zeros, whose keys differ
+  // though they sort as equal; ranks are then the sorted order.
+  bool sorted = false;
+  if (k <= kBoundMaxK && staged) {
+    constexpr int kSample = (2 * kBoundMaxK + kSampleMaxCols / kSliceLen + 63) / 64;
+    __shared__ __attribute__((aligned(16))) unsigned s_few[kBoundMaxKeys + 16];
+    __shared__ unsigned s_at[kBoundMaxKeys];
+    const int first = min(k, (2 * k + a.slices - 1) / a.slices), lane = tid & 63;
+    unsigned b[kSample];
+#pragma unroll
+    for (int r = 0; r < kSample; ++r) {
+      const int i = lane + 64 * r;
+      b[r] = i < first * a.slices ? s_cand[i / first * k + i % first] : 0u;
     }
-  }
-  unsigned total;
-  const unsigned at = BlockScan<kPickThreads>(counts, s_wave, &total);
-  unsigned up = at >> kUpShift, eq = at & kEqMask;
-  for (int j = 0; j < per; ++j) {
-    const int i = i0 + j;
-    if (i >= n)
-      break;
-    const unsigned key = key_of(i);
-    if (key > kth) {
-      s_val[up] = cv[i];
-      s_idx[up] = ci[i];
-      ++up;
-    } else if (key == kth) {
-      if (eq < ties) {
-        s_val[unsigned(k) - ties + eq] = cv[i];
-        s_idx[unsigned(k) - ties + eq] = ci[i];
-      }
-      ++eq;
-    }
-  }
-  __syncthreads();
-  // Bitonic sort of the k winners: value descending, index ascending. Up to
-  // 64 winners sort in one wave's registers (lane p holds position p;
-  // exchanges by lane shuffles, no barriers); more sort in LDS.
-  int size = 1;
-  while (size < k)
-    size <<= 1;
-  if (size <= 64) {
-    if (tid < 64) {
-      float v = tid < k ? s_val[tid] : -INFINITY;
-      unsigned ix = tid < k ? s_idx[tid] : kPadIndex;
-      for (int len = 2; len <= 64; len <<= 1)
-        for (int stride = len >> 1; stride > 0; stride >>= 1) {
-          const float ov = __shfl_xor(v, stride, 64);
-          const unsigned oi = unsigned(__shfl_xor(int(ix), stride, 64));
-          // The lower lane of a pair keeps the first of the two in an
-          // ascending run ((p & len) == 0), the upper lane in a descending one.
-          const bool wants_first = ((tid & stride) == 0) == ((tid & len) == 0);
-          const bool mine_first = v > ov || (v == ov && ix < oi);
-          if (wants_first != mine_first) {
-            v = ov;
-            ix = oi;
+    const unsigned bound = KeyBound(b, k);
+    if (bound > 0x80000000u) {  // uniform
+      unsigned own = 0, found;
+      for (int j = 0; j < per; ++j)
+        own += i0 + j < n && s_cand[i0 + j] >= bound ? 1u : 0u;
+      unsigned at = BlockScan<kPickThreads>(own, s_wave, &found);
+      if (found <= unsigned(kBoundMaxKeys)) {  // uniform
+        if (tid < 16)
+          s_few[found + tid] = 0u;
+        for (int j = 0; j < per; ++j)
+          if (i0 + j < n && s_cand[i0 + j] >= bound) {
+            s_few[at] = s_cand[i0 + j];
+            s_at[at] = s_ci[i0 + j];
+            ++at;
           }
-        }
-      if (tid < k) {
-        s_val[tid] = v;
-        s_idx[tid] = ix;
-      }
-    }
-    __syncthreads();
-  } else {
-    for (int i = k + tid; i < size; i += kPickThreads) {
-      s_val[i] = -INFINITY;
-      s_idx[i] = kPadIndex;
-    }
-    __syncthreads();
-    const auto first = [&](int p, int q) {
-      return s_val[p] > s_val[q] || (s_val[p] == s_val[q] && s_idx[p] < s_idx[q]);
-    };
-    for (int len = 2; len <= size; len <<= 1)
-      for (int stride = len >> 1; stride > 0; stride >>= 1) {
-        for (int i = tid; i < size; i += kPickThreads) {
-          const int j = i ^ stride;
-          if (j > i && ((i & len) == 0 ? first(j, i) : first(i, j))) {
-            const float tv = s_val[i];
-            s_val[i] = s_val[j];
-            s_val[j] = tv;
-            const unsigned ti = s_idx[i];
-            s_idx[i] = s_idx[j];
-            s_idx[j] = ti;
+        __syncthreads();
+        for (int j = tid; j < int(found); j += kPickThreads) {
+          const int rank = RankOf(s_few, int(found), j);
+          if (rank < k) {
+            s_val[rank] = OrderedValue(s_few[j]);
+            s_idx[rank] = s_at[j];
           }
         }
         __syncthreads();
+        sorted = true;
       }
+    }
+  }
+  if (!sorted) {
+    unsigned kth, ties;
+    SelectKth<kPickThreads>(n, unsigned(k), key_of, s_hist, s_sel, kth, ties);
+    // Counts, one block scan, then the winners in order.
+    unsigned counts = 0;
+    for (int j = 0; j < per; ++j) {
+      const int i = i0 + j;
+      if (i < n) {
+        const unsigned key = key_of(i);
+        counts += key > kth ? (1u << kUpShift) : key == kth ? 1u : 0u;
+      }
+    }
+    unsigned total;
+    const unsigned at = BlockScan<kPickThreads>(counts, s_wave, &total);
+    unsigned up = at >> kUpShift, eq = at & kEqMask;
+    for (int j = 0; j < per; ++j) {
+      const int i = i0 + j;
+      if (i >= n)
+        break;
+      const unsigned key = key_of(i);
+      if (key > kth) {
+        s_val[up] = cv[i];
+        s_idx[up] = ci[i];
+        ++up;
+      } else if (key == kth) {
+        if (eq < ties) {
+          s_val[unsigned(k) - ties + eq] = cv[i];
+          s_idx[unsigned(k) - ties + eq] = ci[i];
+        }
+        ++eq;
+      }
+    }
+    __syncthreads();
+    // Bitonic sort of the k winners: value descending, index ascending. Up to
+    // 64 winners sort in one wave's registers (lane p holds position p;
+    // exchanges by lane shuffles, no barriers); more sort in LDS.
+    int size = 1;
+    while (size < k)
+      size <<= 1;
+    if (size <= 64) {
+      if (tid < 64) {
+        float v = tid < k ? s_val[tid] : -INFINITY;
+        unsigned ix = tid < k ? s_idx[tid] : kPadIndex;
+        for (int len = 2; len <= 64; len <<= 1)
+          for (int stride = len >> 1; stride > 0; stride >>= 1) {
+            const float ov = __shfl_xor(v, stride, 64);
+            const unsigned oi = unsigned(__shfl_xor(int(ix), stride, 64));
+            // The lower lane of a pair keeps the first of the two in an
+            // ascending run ((p & len) == 0), the upper lane in a descending one.
+            const bool wants_first = ((tid & stride) == 0) == ((tid & len) == 0);
+            const bool mine_first = v > ov || (v == ov && ix < oi);
+            if (wants_first != mine_first) {
+              v = ov;
+              ix = oi;
+            }
+          }
+        if (tid < k) {
+          s_val[tid] = v;
+          s_idx[tid] = ix;
+        }
+      }
+      __syncthreads();
+    } else {
+      for (int i = k + tid; i < size; i += kPickThreads) {
+        s_val[i] = -INFINITY;
+        s_idx[i] = kPadIndex;
+      }
+      __syncthreads();
+      const auto first = [&](int p, int q) {
+        return s_val[p] > s_val[q] || (s_val[p] == s_val[q] && s_idx[p] < s_idx[q]);
+      };
+      for (int len = 2; len <= size; len <<= 1)
+        for (int stride = len >> 1; stride > 0; stride >>= 1) {
+          for (int i = tid; i < size; i += kPickThreads) {
+            const int j = i ^ stride;
+            if (j > i && ((i & len) == 0 ? first(j, i) : first(i, j))) {
+              const float tv = s_val[i];
+              s_val[i] = s_val[j];
+              s_val[j] = tv;
+              const unsigned ti = s_idx[i];
+              s_idx[i] = s_idx[j];
+              s_idx[j] = ti;
+            }
+          }
+          __syncthreads();
+        }
+    }
   }
   // The weights in parallel (the sorted maximum first), then the running
   // sums in candidate order on one thread.
@@ -583,22 +761,36 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   for (int i = tid; i < k; i += kPickThreads)
     s_w[i] = expf((s_val[i] - top) * a.inv_t);
   __syncthreads();
+  // The running sums in candidate order on one thread (the last is the
+  // total), then the first candidate with weight whose sum passes the
+  // target, or the last with weight should the sums round.
+  __shared__ float s_run[kSampleMaxTopK];
   if (tid == 0) {
     float total = 0.0f;
-    for (int i = 0; i < k; ++i)
-      total += s_w[i];
-    const float target = u * total;
-    float run = 0.0f;
-    int pick = 0;
+#pragma unroll 8
     for (int i = 0; i < k; ++i) {
-      const float w = s_w[i];
-      if (w > 0.0f)
-        pick = i;  // the last candidate with weight, should the sums round
-      run += w;
-      if (w > 0.0f && run > target)
-        break;
+      total += s_w[i];
+      s_run[i] = total;
     }
-    a.ids[row] = s_idx[pick];
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const float target = u * s_run[k - 1];
+    int pick = 0;
+    for (int i0 = 0; i0 < k; i0 += 64) {
+      const int i = i0 + tid;
+      const bool weighs = i < k && s_w[i] > 0.0f;
+      const unsigned long long all = __ballot(weighs);
+      const unsigned long long past = __ballot(weighs && s_run[i] > target);
+      if (past) {
+        pick = i0 + __ffsll((long long)past) - 1;
+        break;
+      }
+      if (all)
+        pick = i0 + 63 - __clzll((long long)all);
+    }
+    if (tid == 0)
+      a.ids[row] = s_idx[pick];
   }
 }
 

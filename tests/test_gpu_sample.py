@@ -215,3 +215,40 @@ def test_engine_sampled_round_matches_lfm3_sample():
     for s in a + b:
         s.close()
     gm.close()
+
+
+def special_rows(kind, V):
+    x = rows_of(f"sample.bound.{kind}.{V}", 4, V, 3.0)
+    if kind == "equal":        # more equal keys than the bounded path holds
+        x[:] = 1.5
+        x[1, V // 2] = 2.0
+        x[2, : V // 2] = 1.75
+    elif kind == "ties":       # a tie at the k-th value in every slice, and across slices
+        x = np.minimum(np.round(x * 2) / 2, 6.0).astype(np.float32)
+    elif kind == "negative":   # no logit above zero, the largest in every slice zeros
+        x = -np.abs(x) - 0.5
+        x[:2, ::97] = 0.0
+        x[2:, ::97] = np.float32(-0.0)
+    elif kind == "infinite":   # masked tokens, the type's lowest value, one huge leader
+        x[:, ::2] = -np.inf
+        x[:, 1::6] = np.finfo(np.float32).min
+        x[3, 11] = 1e30
+    return np.ascontiguousarray(x)
+
+
+@pytest.mark.parametrize("kind", ["plain", "equal", "ties", "negative", "infinite"])
+@pytest.mark.parametrize("V,k", [(9000, 2), (9000, 128), (9000, 129), (4096, 64), (70000, 50),
+                                 (4200, 100)])
+def test_top_k_edges_match_the_oracle(kind, V, k):
+    """Top-k where the bounded selection starts and ends (k up to 128, at
+    most 512 keys at or above the bound, a bound above zero, slices shorter
+    than k) and where the radix select takes over: the oracle's picks over a
+    grid of uniforms."""
+    x = special_rows(kind, V)
+    grid = np.linspace(0.0, 0.999, 16, dtype=np.float32)
+    for r in range(x.shape[0]):
+        rows = np.repeat(x[r:r + 1], len(grid), axis=0)
+        got = sample(rows, 0.9, k, u=grid)
+        for g, u in zip(got, grid):
+            want = O.sample(x[r], 0.9, k, 1.0, None, float(u))
+            assert g == want or consistent(x[r], 0.9, k, 1.0, None, float(u), int(g)), (r, u, g, want)
