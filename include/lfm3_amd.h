@@ -591,11 +591,13 @@ int lfm3_pack_kv(const float* k, const float* v, uint16_t* k16, uint16_t* v16,
 int lfm3_store_kv(const uint16_t* k16, const uint16_t* v16, uint16_t* cache_k,
                   uint16_t* cache_v, uint32_t rows, uint32_t stride,
                   uint32_t position, uint32_t capacity, void* stream);
-/* Workspace of lfm3_prompt_attention: key spans of long global histories
-   (whole 64-key tiles, at least 1024 keys each, at most 16, as many as
-   bring the launch to about one block per CU) keep partial sums, rows x
-   heads x (dim + 2) floats a span; this bounds any head grouping. 0 when
-   the keys fit one span or window > 0. */
+/* Workspace of lfm3_prompt_attention: key spans of global histories from
+   640 keys on (whole 64-key tiles, at least 256 keys each, as many as one
+   round of blocks on the CUs takes, at most 16) keep partial sums, rows x
+   heads x (dim + 2) floats a span; this bounds any head grouping and
+   serves every call of fewer rows. 0 when the keys fit one span or window
+   > 0. A smaller workspace makes fewer spans; spans of at least 1024 keys
+   have to fit. */
 size_t lfm3_prompt_attention_workspace_bytes(uint32_t rows, uint32_t heads,
                                              uint32_t dim, uint32_t position,
                                              uint32_t window);
@@ -623,7 +625,8 @@ int lfm3_prompt_attention(const float* q, uint32_t ldq, const uint16_t* k,
 /* lfm3_prompt_attention with its output written as the output projection's
    FP16 row-scaled activations: row r's heads * dim outputs (the same FP32
    values) go to out + r * lda as fp16(out 2^e) with scale[r] = 2^-e, e =
-   14 - ilogb(max |row|) (lfm3_half_rows of the FP32 output, bit for bit).
+   14 - ilogb(max |row|) (lfm3_half_rows of the FP32 output, bit for bit
+   where both calls have the workspaces their functions give).
    Every call keeps per-span partial sums in the workspace
    (lfm3_prompt_attention_half_workspace_bytes, at least one span); a
    per-row merge writes the rows. lda % 64 == 0, lda >= heads * dim.

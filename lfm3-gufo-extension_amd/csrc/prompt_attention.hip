@@ -26,10 +26,11 @@
 // never cross lanes. A column's softmax state is per lane; its row maximum
 // and final sum combine the 4 lanes of the column (L % 16) with two
 // exchanges. Long global histories split keys across blockIdx.y into spans
-// (SpanPlan: enough spans for about one block per CU, whole 64-key tiles,
-// at least 1024 keys and at most 16 spans; the reference's PromptSplits
+// (SpanPlan: as many spans as one round of blocks takes, whole 64-key tiles,
+// at least 256 keys and at most 16 spans; the reference's PromptSplits
 // instead fixes spans of at least 2048 keys, at most 8). Each span stores
 // its maximum, sum and unnormalized output, merged by CombineSpansKernel.
+#include <algorithm>
 #include <cmath>
 
 #include "common.hpp"
@@ -40,17 +41,27 @@ namespace {
 constexpr int kPAWaves = 8, kPAThreads = 64 * kPAWaves;
 constexpr int kPAKeys = 64;             // keys a tile
 
-// Key spans of a long causal history (blockIdx.y of the tile launch): a
-// launch of row blocks x KV heads blocks per span is cut into spans until
-// it has about one block per CU, each span a whole number of 64-key tiles
-// and at least kSpanFloorTiles tiles long, so the merge launch stays small
-// next to the spans. A sliding window never splits.
-constexpr int kFillBlocks = 256, kSpanFloorTiles = 16, kMaxSpans = 16;
+// Key spans of a causal history (blockIdx.y of the tile launch): as many as
+// fill the CUs without a second round of blocks, each a whole number of
+// 64-key tiles and at least kSpanFloorTiles long. A block takes about 1.9 us
+// a tile, most of it latency at two waves a SIMD, whatever the CUs beside it
+// do: the attention call of 77 rows after 3000 takes 35.8 us in spans of at
+// least 16 tiles and 20.0 of 4, 512 rows after 1000 49.4 and 25.3; 300 rows
+// after 3000 40.8 in 3 spans, 30.0 in 6 and 37 in 13 (a second round). More
+// than 16 spans cost the merge what they save (30 rows after 20000 41.5 us
+// in 16, 43.3 in 32). Histories under kSplitTiles (640 keys) and sliding
+// windows never split.
+constexpr int kSpanFloorTiles = 4, kSplitTiles = 10, kMaxSpans = 16;
 
-int SpanPlan(int keys, int blocks_per_span, int& span_keys) {
+// Spans at most for so many tiles.
+int TileSpans(int tiles) {
+  return tiles < kSplitTiles ? 1 : std::min(kMaxSpans, tiles / kSpanFloorTiles);
+}
+
+int SpanPlan(int keys, int blocks_per_span, int fill, int room, int& span_keys) {
   const int tiles = (keys + kPAKeys - 1) / kPAKeys;
-  int spans = (kFillBlocks + blocks_per_span - 1) / std::max(blocks_per_span, 1);
-  spans = std::min({spans, kMaxSpans, std::max(1, tiles / kSpanFloorTiles)});
+  const int spans = std::max(
+      1, std::min({fill / std::max(blocks_per_span, 1), TileSpans(tiles), room}));
   span_keys = (tiles + spans - 1) / spans * kPAKeys;
   return (keys + span_keys - 1) / span_keys;
 }
@@ -552,24 +563,44 @@ struct PromptArgs {
 };
 
 // Long histories: two column tiles a wave (each K / V operand read feeds two
-// MFMAs); windows and short histories: one, for more blocks.
-int ColumnTiles(int position, int n, int window) {
-  return window == 0 && position + n > 4096 ? 2 : 1;
+// MFMAs); windows and short histories, and rows that one column tile a wave
+// holds: one, for more blocks or fewer empty columns.
+int ColumnTiles(int position, int n, int window, int group) {
+  return window == 0 && position + n > 4096 && n * group > 16 * kPAWaves ? 2 : 1;
 }
 
 // The span plan of one call: span length and count for the tile launch of
-// the chosen shape (spans > 1 only for a history without a window).
-int PlanCall(int n, int position, int window, int group, int kv_heads, int& span) {
+// the chosen shape (spans > 1 only for a history without a window), at most
+// `room` spans where the workspace holds no more.
+int PlanCall(int n, int position, int window, int group, int kv_heads, int dim, int room,
+             int& span) {
   const int keys = position + n;
   span = keys;
   if (window)
     return 1;
-  const int rows = 16 * ColumnTiles(position, n, window) * kPAWaves / group;
+  const int column_tiles = ColumnTiles(position, n, window, group);
+  const int rows = 16 * column_tiles * kPAWaves / group;
   const int blocks_per_span = (n + rows - 1) / rows * kv_heads;
-  const int spans = SpanPlan(keys, blocks_per_span, span);
+  // Blocks a round: two a CU where 64 dimensions and one column tile leave
+  // the registers (300 rows after 3000 of 32 x 64 heads 69.6 us against 71.4).
+  const int fill = dim == 64 && column_tiles == 1 ? 512 : 256;
+  const int spans = SpanPlan(keys, blocks_per_span, fill, room, span);
   if (spans == 1)
     span = keys;
   return spans;
+}
+
+// Spans that a call's workspace has to hold: spans of at least 1024 keys, at
+// most 16, for about one block a CU of the larger block. A workspace between
+// this and the plan's own need takes fewer spans.
+int LeastSpans(int n, int position, int window, int group, int kv_heads) {
+  if (window)
+    return 1;
+  const int keys = position + n, rows = 16 * (keys > 4096 ? 2 : 1) * kPAWaves / group;
+  const int blocks = (n + rows - 1) / rows * kv_heads, tiles = (keys + kPAKeys - 1) / kPAKeys;
+  const int spans = std::min({(256 + blocks - 1) / blocks, kMaxSpans, std::max(1, tiles / 16)});
+  const int span_tiles = (tiles + spans - 1) / spans;
+  return (tiles + span_tiles - 1) / span_tiles;
 }
 
 template<int D, int G, int CT>
@@ -588,7 +619,7 @@ void LaunchTiles(const PromptArgs& a, hipStream_t s) {
 
 template<int D, int G>
 void LaunchPrompt(const PromptArgs& a, hipStream_t s) {
-  if (ColumnTiles(a.position, a.n, a.window) == 2)
+  if (ColumnTiles(a.position, a.n, a.window, G) == 2)
     LaunchTiles<D, G, 2>(a, s);
   else
     LaunchTiles<D, G, 1>(a, s);
@@ -616,8 +647,7 @@ void LaunchPromptGroup(const PromptArgs& a, int group, hipStream_t s) {
 int MostSpans(std::uint32_t position, std::uint32_t n, std::uint32_t window) {
   if (window)
     return 1;
-  const int tiles = int((std::uint64_t(position) + n + kPAKeys - 1) / kPAKeys);
-  return std::min(kMaxSpans, std::max(1, tiles / kSpanFloorTiles));
+  return TileSpans(int((std::uint64_t(position) + n + kPAKeys - 1) / kPAKeys));
 }
 
 }  // namespace
@@ -673,12 +703,16 @@ int PromptAttention(const float* q, std::uint32_t ldq, const std::uint16_t* k,
       !BufferFits(std::size_t(capacity) * kv_heads * dim * 2))
     return Fail(LFM3_E_INVALID, "unsupported LFM3 prompt attention shape");
   PromptArgs a{};
-  a.splits = PlanCall(int(rows), int(position), int(window), int(group), int(kv_heads), a.span);
-  const std::size_t need = a.splits > 1 || half
-                               ? std::size_t(a.splits) * rows * heads * (dim + 2) * sizeof(float)
-                               : 0;
+  // A span's partials.
+  const std::size_t span_bytes = std::size_t(rows) * heads * (dim + 2) * sizeof(float);
+  const int least = LeastSpans(int(rows), int(position), int(window), int(group), int(kv_heads));
+  const std::size_t need = least > 1 || half ? least * span_bytes : 0;
   if (need && (!workspace || workspace_bytes < need))
     return Fail(LFM3_E_INVALID, "LFM3 prompt attention workspace too small");
+  const int room = int(std::min<std::size_t>(workspace ? workspace_bytes / span_bytes : 1,
+                                             kMaxSpans));
+  a.splits = PlanCall(int(rows), int(position), int(window), int(group), int(kv_heads), int(dim),
+                      room, a.span);
   a.q = q;
   a.ldq = int(ldq);
   a.k = k;

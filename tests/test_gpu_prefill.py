@@ -448,3 +448,64 @@ def test_prompt_attention_strided_rows_from_projection():
     dense, _ = run_prompt_attention(q, gates, kbits, vbits, ckbits, cvbits, n, H, KH, D, P,
                                     P + n, 0)
     assert np.array_equal(strided, dense)
+
+
+@pytest.mark.parametrize("n,P,H,KH,D", [
+    (1, 639, 16, 4, 128),      # ten tiles: the first length that splits
+    (30, 9000, 16, 4, 128),    # few rows after a long history: one column tile a wave
+    (33, 9000, 16, 4, 128),    # two column tiles, a row past the smaller block
+    (128, 2500, 4, 2, 128),    # spans of four tiles
+    (40, 8200, 32, 8, 64),     # two blocks a CU of the 64-dimension heads
+])
+def test_prompt_attention_span_plans(n, P, H, KH, D):
+    """Histories cut into few and into many spans, at the edges of the plan:
+    the FP32 rows within the gate of the FP64 formula, the FP16 rows the
+    same values, and with the least workspace (spans of at least 1024 keys,
+    at most 16) the same rows but for the order of the spans' sums."""
+    tag = f"{n}.{P}.{H}.{D}"
+    stride, cap = KH * D, P + n
+    q = L.normal(SEED, f"psp.q.{tag}", n * H * D).reshape(n, H * D)
+    gates = L.normal(SEED, f"psp.g.{tag}", n * H).reshape(n, H)
+    bits = [L.half_normal(SEED, f"psp.{t}.{tag}", r * stride)
+            for t, r in (("k", n), ("v", n), ("ck", cap), ("cv", cap))]
+    out, ws_bytes = run_prompt_attention(q, gates, *bits, n, H, KH, D, P, cap, 0)
+    span = n * H * (D + 2) * 4
+    assert ws_bytes > span and ws_bytes % span == 0
+    want = prompt_attention_fp64(q, gates, *[O.half_to_float(b) for b in bits], n, H, KH, D, P,
+                                 cap, 0)
+    assert np.max(np.abs(out - want)) < 1e-3
+    dq, dg = L.DeviceBuffer.of(np.ascontiguousarray(q)), L.DeviceBuffer.of(gates)
+    dev = [L.DeviceBuffer.of(b) for b in bits]
+    least = min(16, max(1, (P + n + 63) // 64 // 16))
+
+    def half(spans_bytes):
+        ws = L.DeviceBuffer(spans_bytes)
+        da, ds = L.DeviceBuffer(n * H * D * 2), L.DeviceBuffer(n * 4)
+        L.check(L.lib().lfm3_prompt_attention_half(
+            dq.addr, H * D, dev[0].addr, dev[1].addr, dg.addr, H, dev[2].addr, dev[3].addr,
+            da.addr, H * D, ds.addr, n, H, KH, D, P, cap, 0, ws.addr, spans_bytes, None))
+        L.synchronize()
+        return (da.download(np.uint16, n * H * D).reshape(n, H * D), ds.download(np.float32, n))
+
+    assert L.lib().lfm3_prompt_attention_half_workspace_bytes(n, H, D, P, 0) == ws_bytes
+    a, scale = half(ws_bytes)
+    _, exps = O.half_rows(out)
+    assert np.array_equal(a, O.float_to_half(np.ldexp(out, exps[:, None]).astype(np.float32)))
+    assert np.array_equal(scale, np.ldexp(np.float32(1), -exps).astype(np.float32))
+    b, bscale = half(least * span)
+    rows = O.half_to_float(b.reshape(-1)).reshape(n, H * D) * bscale[:, None]
+    assert np.max(np.abs(rows - want)) < 1e-3
+
+
+def test_prompt_attention_workspace_serves_fewer_rows():
+    """A workspace sized for some rows and position holds every call of
+    fewer, and none is asked for where nothing splits."""
+    f = L.lib().lfm3_prompt_attention_workspace_bytes
+    h = L.lib().lfm3_prompt_attention_half_workspace_bytes
+    for P in (0, 500, 2000, 24000, 262144):
+        sizes = [h(n, 16, 128, P, 0) for n in range(1, 700)]
+        assert all(x <= y for x, y in zip(sizes, sizes[1:]))
+    for n in (1, 77, 512):
+        sizes = [h(n, 16, 128, P, 0) for P in range(0, 30000, 61)]
+        assert all(x <= y for x, y in zip(sizes, sizes[1:]))
+    assert f(64, 16, 128, 500, 0) == 0 and f(512, 16, 128, 24576, 256) == 0
