@@ -11,11 +11,22 @@
 // holds each query head as an fp16 hi row and an fp16 lo row (hi + lo 2^-11
 // keeps about 22 bits of the FP32 query; every half x half product is
 // exact in FP32), the B operand is 16 keys' F16 rows read with one 16-byte
-// load per lane per 32 dimensions. The softmax runs in (head, key) lanes
-// with FP32 online maxima and sums; P V runs on the VALU, a lane owning
-// eight dimensions of a quarter of the group's keys (one 16-byte V load per
-// key), with the probabilities broadcast through LDS. The next group's K
-// and V loads are issued before the current group is computed. Waves merge
+// load per lane per 32 dimensions. The A rows are ordered so that a lane's
+// product holds the hi and lo sums of its own (head, key): the base-2 online
+// softmax starts in those registers, with FP32 maxima and each lane's own
+// sums. P V runs on the VALU (v_fma_mix, the F16 value read in place), a lane
+// owning eight dimensions of a quarter of the group's keys (one 16-byte V
+// load per key), with the probabilities broadcast through LDS. The next
+// group's K and V loads are issued before the current group is computed.
+// What bounds a long span is the chain of one group (products, maximum,
+// exponential, the exchange, P V) at two or three waves a SIMD beside the
+// loads, and a short one the launch's fixed chain. Dropping the scores' own
+// LDS exchange, a division, two conversions a value and the current key's
+// selects, and building the query operand without a branch a read, took one
+// row of 131072 keys from 68.2 to 61.2 us (4.4 TB/s), 8 rows of 128 to 8192
+// keys from 21.0 to 19.3, 8 rows of 16K-32K from 91.6 to 88.3, 8 sliding
+// rows from 9.0 to 8.3. Eight waves a block in 128 registers: 59.2 us for
+// the one row, 102 for the eight of 16K-32K. Waves merge
 // through LDS; rows with several spans leave per-span (max, sum, acc)
 // partials, and the last span block of a (row, KV head) to arrive merges
 // them in span order, so results do not depend on block scheduling. The
@@ -32,9 +43,9 @@
 // norms and rotations compute. Exactly one block of a row writes the
 // ring: the one whose span ends at the current position. It stores the
 // row's F16 K/V to slot position % capacity for later rounds and takes
-// that key from LDS for this one (the ring loads skip it, and the group
-// holding it selects the LDS row in its place), so nothing waits for the
-// store. No other span of the row covers the current position, so no
+// that key from LDS for this one (the ring loads skip it; its score and
+// value row enter the merge of the waves as an entry of their own), so
+// nothing waits for the store. No other span of the row covers the current position, so no
 // other block reads the slot being written; on a sliding layer this
 // relies on the ring holding at least the window (capacity = min(context,
 // window) >= keys of any span), so the current slot is not an earlier key
@@ -84,7 +95,7 @@ __device__ __forceinline__ float AgentLoad(const float* p) {
 template<int D, int G, int T>
 __device__ void MergeSpans(const lfm3_attention_item& item, int g, int kv_heads,
                            const float* partial, const float* s_gate, float* out, int ldo,
-                           float (*s_w)[G], float (*s_lv)[G], float* s_top, float* s_den) {
+                           float (*s_w)[G], float (*s_lv)[G], float* s_den) {
   const int row = int(item.row), parts = int(item.parts), tid = threadIdx.x;
   const std::size_t span_stride = std::size_t(kv_heads) * G * (D + 2);
   const float* base = partial + (std::size_t(item.first_item) * kv_heads + g) * G * (D + 2);
@@ -95,29 +106,27 @@ __device__ void MergeSpans(const lfm3_attention_item& item, int g, int kv_heads,
     s_lv[s][h] = AgentLoad(po + 1);
   }
   __syncthreads();
-  if (tid < G) {
-    float top = -INFINITY;
-    for (int s = 0; s < parts; ++s)
-      top = fmaxf(top, s_w[s][tid]);
-    s_top[tid] = top;
-  }
-  __syncthreads();
-  for (int e = tid; e < parts * G; e += T) {
-    const int s = e / G, h = e % G;
-    s_w[s][h] = expf(s_w[s][h] - s_top[h]);
-  }
-  __syncthreads();
-  if (tid < G) {
-    float den = 0.0f;
-    for (int s = 0; s < parts; ++s)
-      den = fmaf(s_lv[s][tid], s_w[s][tid], den);
-    s_den[tid] = den;
+  // A wave a head: the spans' top, weights and denominator over its lanes.
+  for (int h = tid >> 6; h < G; h += T / 64) {
+    float top = -INFINITY, den = 0.0f;
+    for (int s = tid & 63; s < parts; s += 64)
+      top = fmaxf(top, s_w[s][h]);
+    top = WaveMax(top);
+    for (int s = tid & 63; s < parts; s += 64) {
+      const float w = __builtin_amdgcn_exp2f(s_w[s][h] - top);
+      den = fmaf(s_lv[s][h], w, den);
+      s_w[s][h] = w;
+    }
+    den = WaveSum(den);
+    if ((tid & 63) == 0)
+      s_den[h] = den;
   }
   __syncthreads();
   // Every element's sum first, then the stores. The loads of kBatch spans
   // of every element a thread owns go out together (one memory round trip
   // a batch); the sums then run in span order. A batch's loads past the
-  // last span repeat the last one and are not added.
+  // last span repeat the last one and are not added. (Batches of 32: 63.0
+  // us against 61.6 for 128 spans, 19.1 against 18.2 for 44.)
   constexpr int EPT = (G * D + T - 1) / T, kBatch = 16;
   float av[EPT];
   const float* po[EPT];
@@ -184,14 +193,15 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
   static_assert(D == 64 || D == 128, "head dimension 64 or 128");
   static_assert(2 * G <= 16, "hi and lo rows of the group fit one MFMA tile");
   constexpr int S = D / 32;                // MFMA steps per key row
-  constexpr int PAIRS = (16 * G + 63) / 64;
-  __shared__ float s_q[G][D];
+  // Lane L's scores: key L % 16 of heads HPL (L / 16) .. + HPL - 1.
+  constexpr int HPL = G > 4 ? G / 4 : 1;
+  __shared__ __attribute__((aligned(16))) float s_q[G][D];
   __shared__ __attribute__((aligned(16))) Half s_kv[2][D];
-  __shared__ float s_tile[NW][16][17];
-  __shared__ float s_p[NW][kGroupKeys][G];
-  __shared__ float s_alpha[NW][G];
+  __shared__ __attribute__((aligned(16))) float s_p[NW][kGroupKeys][G];
+  __shared__ __attribute__((aligned(16))) float s_alpha[NW][G];
   __shared__ __attribute__((aligned(16))) float s_acc[NW][G][D];
-  __shared__ float s_m[NW][G], s_l[NW][G];
+  // Each wave's maximum and sum; the last maximum: the current key's score.
+  __shared__ float s_m[NW + 1][G], s_l[NW][G];
   __shared__ float s_gate[G];
 
   const lfm3_attention_item item = items[blockIdx.x];
@@ -221,43 +231,47 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
   const BufferResource k_res = MakeBuffer(ck, ring_bytes);
   const BufferResource v_res = MakeBuffer(cv, ring_bytes);
   const int n = lane & 15, kg = lane >> 4;
-  // Ring slots of keys base + o (o < 16) for the lane's K row (o = n) and V
-  // rows (o = kq + KG i): one wave-uniform division per group, then the
-  // wrap as an unsigned minimum (rings of 16 slots or more; smaller rings
-  // take the remainder). Keys past the span, and groups past the wave's
-  // last, read zeros from an offset the hardware drops (no traffic). The
-  // offsets are selects, not branches around the loads.
-  const int ngroups = ngroups_of(kb, ke);
+  // Byte offsets of keys base + o (o < 16) for the lane's K row (o = n) and
+  // V rows (o = kq + KG i): the ring offset of the wave's next group (uniform,
+  // advanced by the waves' groups) plus the lane's, wrapped as an unsigned
+  // minimum (rings of 16 slots or more; smaller rings take the remainder).
+  // Keys past the span, and groups past the wave's last, read zeros from an
+  // offset the hardware drops (no traffic). The offsets are selects, not
+  // branches around the loads.
+  const int keys = ke - held;  // the keys read through the ring end here
+  const int ngroups = ngroups_of(kb, keys);
   const unsigned row_bytes = unsigned(stride) * 2;
   const unsigned k_lane = unsigned(g * D + 8 * kg) * 2, v_lane = unsigned(g * D + 8 * dg) * 2;
+  const unsigned k_at = unsigned(n) * row_bytes + k_lane, v_at = unsigned(kq) * row_bytes + v_lane;
+  unsigned slot = unsigned(kb + kGroupKeys * wave) % cap;  // of the next group's first key
   const auto fetch = [&](int j, uint4 (&kr)[S], uint4 (&vr)[KPL]) {
-    const int base = kb + kGroupKeys * j;
-    // Keys of the group inside the span; the current position's key (the
-    // span's last when it holds it) comes from LDS instead (patch below).
-    const int rem = j < ngroups ? ke - held - base : 0;
-    const unsigned b0 = unsigned(base) % cap;
-    unsigned sk = b0 + unsigned(n), sv[KPL];
+    const int rem = j < ngroups ? keys - (kb + kGroupKeys * j) : 0;
+    const unsigned b0 = slot * row_bytes;
+    unsigned koff = b0 + k_at, voff[KPL];
 #pragma unroll
     for (int i = 0; i < KPL; ++i)
-      sv[i] = b0 + unsigned(kq + KG * i);
+      voff[i] = b0 + v_at + unsigned(KG * i) * row_bytes;
     if (cap >= 16) {
-      sk = min(sk, sk - cap);
+      koff = min(koff, koff - ring_bytes);
 #pragma unroll
       for (int i = 0; i < KPL; ++i)
-        sv[i] = min(sv[i], sv[i] - cap);
+        voff[i] = min(voff[i], voff[i] - ring_bytes);
     } else {
-      sk %= cap;
+      koff = (slot + unsigned(n)) % cap * row_bytes + k_lane;
 #pragma unroll
       for (int i = 0; i < KPL; ++i)
-        sv[i] %= cap;
+        voff[i] = (slot + unsigned(kq + KG * i)) % cap * row_bytes + v_lane;
     }
-    const unsigned koff = n < rem ? sk * row_bytes + k_lane : kOutOfRange;
+    koff = n < rem ? koff : kOutOfRange;
 #pragma unroll
     for (int s2 = 0; s2 < S; ++s2)
       kr[s2] = LoadB128(k_res, koff + 64 * s2);
 #pragma unroll
     for (int i = 0; i < KPL; ++i)
-      vr[i] = LoadB128(v_res, kq + KG * i < rem ? sv[i] * row_bytes + v_lane : kOutOfRange);
+      vr[i] = LoadB128(v_res, kq + KG * i < rem ? voff[i] : kOutOfRange);
+    slot += unsigned(kGroupKeys * NW);
+    if (slot >= cap)
+      slot = cap >= unsigned(kGroupKeys * NW) ? slot - cap : slot % cap;
   };
 
   uint4 kr[S], vr[KPL];
@@ -359,26 +373,59 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
     __syncthreads();
   }
 
-  // A operand: row m < G is head m's hi part, G <= m < 2G head m - G's lo.
-  h8 a[S];
-  {
-    const int m = lane & 15, kg = lane >> 4;
-    const int head = m < G ? m : m < 2 * G ? m - G : 0;
+  // The scores in units of log2: exp2 in place of exp, and no division.
+  const float scale = 1.44269504088896341f / sqrtf(float(D));
+  if constexpr (kFused) {
+    // The current position's key, a wave a head: an entry of its own in the
+    // merge of the waves (its F16 row is in LDS; nothing in the key loop
+    // looks for it).
+    for (int h = wave; held && h < G; h += NW) {
+      float sc = 0.0f;
 #pragma unroll
-    for (int s = 0; s < S; ++s)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float x = s_q[head][32 * s + 8 * kg + i];
-        const _Float16 hi = static_cast<_Float16>(x);
-        const _Float16 lo = static_cast<_Float16>((x - float(hi)) * 2048.0f);
-        a[s][i] = m < G ? hi : m < 2 * G ? lo : _Float16(0);
-      }
+      for (int d = 0; d < D / 64; ++d)
+        sc = fmaf(s_q[h][lane + 64 * d], HalfBitsToFloat(s_kv[0][lane + 64 * d]), sc);
+      sc = WaveSum(sc);
+      if (lane == 0)
+        s_m[NW][h] = sc * scale;
+    }
   }
 
-  const float root = sqrtf(float(D));
-  float m_own[PAIRS], l_own[PAIRS];
+  // A operand: rows 4 q + 2 r and 4 q + 2 r + 1 are the hi and lo parts of
+  // head HPL q + r, so that lane L of the product holds both sums of its
+  // (head, key) in its own registers.
+  h8 a[S];
+  {
+    const int r = (n & 3) >> 1, h = HPL * (n >> 2) + r;
+    const bool live = r < HPL && h < G;
+    const int head = live ? h : 0;
+    // Read without a condition and masked as bits: as selects of halves the
+    // compiler guarded every read with a branch and waited for each.
+    const unsigned keep = live ? 0xffffffffu : 0u;
 #pragma unroll
-  for (int r = 0; r < PAIRS; ++r) {
+    for (int s = 0; s < S; ++s) {
+      const float4 x0 = *reinterpret_cast<const float4*>(&s_q[head][32 * s + 8 * kg]);
+      const float4 x1 = *reinterpret_cast<const float4*>(&s_q[head][32 * s + 8 * kg + 4]);
+      const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+      unsigned w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        unsigned hi = 0u, lo = 0u;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const unsigned bits = FloatToHalfBits(x[2 * i + j]);
+          const float rest = (x[2 * i + j] - HalfBitsToFloat(bits)) * 2048.0f;
+          hi |= bits << (16 * j);
+          lo |= unsigned(FloatToHalfBits(rest)) << (16 * j);
+        }
+        w[i] = ((n & 1) ? lo : hi) & keep;
+      }
+      a[s] = __builtin_bit_cast(h8, w);
+    }
+  }
+
+  float m_own[HPL], l_own[HPL];  // l_own: the lane's own keys
+#pragma unroll
+  for (int r = 0; r < HPL; ++r) {
     m_own[r] = -INFINITY;
     l_own[r] = 0.0f;
   }
@@ -390,87 +437,73 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
       acc[h][i] = 0.0f;
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 
-  uint4 kn[S], vn[KPL];
-  for (int j = wave; j < ngroups; j += NW) {
-    const int base = kb + kGroupKeys * j;
-    fetch(j + NW, kn, vn);  // past the span: zeros, no traffic
-    if constexpr (kFused) {
-      // The current key (key o of the group holding it; no lane matches in
-      // other groups) from LDS, as selects: a branch here would leave the
-      // compiler's wait counts for the loads in flight inexact, and it
-      // then waits for all of them.
-      const int o = held ? pos - base : -1;
-#pragma unroll
-      for (int s2 = 0; s2 < S; ++s2)
-        kr[s2] = SelectU4(n == o, *reinterpret_cast<const uint4*>(&s_kv[0][32 * s2 + 8 * kg]),
-                          kr[s2]);
-      const uint4 cur_v = *reinterpret_cast<const uint4*>(&s_kv[1][8 * dg]);
-#pragma unroll
-      for (int i = 0; i < KPL; ++i)
-        vr[i] = SelectU4(kq + KG * i == o, cur_v, vr[i]);
-    }
+  const auto step = [&](int j, const uint4 (&kr)[S], const uint4 (&vr)[KPL]) {
     f4 sacc = zero;
 #pragma unroll
     for (int s2 = 0; s2 < S; ++s2)
       sacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s2], __builtin_bit_cast(h8, kr[s2]), sacc, 0, 0, 0);
-    // D layout: lane L holds rows 4 (L / 16) + i of key L % 16.
+    // Online softmax of the lane's key.
+    const bool in_span = kb + kGroupKeys * j + n < keys;
+    bool moved = false;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      s_tile[wave][4 * (lane >> 4) + i][lane & 15] = sacc[i];
-    WaveSync();
-    // Online softmax: lane owns (head, key) pairs idx = lane + 64 r.
-#pragma unroll
-    for (int r = 0; r < PAIRS; ++r) {
-      const int idx = lane + 64 * r, h = idx >> 4, nn = idx & 15;
-      if (h < G) {
-        float sc = (s_tile[wave][h][nn] + s_tile[wave][G + h][nn] * (1.0f / 2048.0f)) / root;
-        if (base + nn >= ke)
-          sc = -INFINITY;
-        const float m_new = fmaxf(m_own[r], GroupMax16(sc));
-        const float shift = m_new == -INFINITY ? 0.0f : m_new;
-        const float p = expf(sc - shift);
-        const float alpha = expf(m_own[r] - shift);
-        l_own[r] = l_own[r] * alpha + GroupSum16(p);
-        m_own[r] = m_new;
-        s_p[wave][nn][h] = p;
-        if (nn == 0)
+    for (int r = 0; r < HPL; ++r) {
+      float sc = (sacc[2 * r] + sacc[2 * r + 1] * (1.0f / 2048.0f)) * scale;
+      sc = in_span ? sc : -INFINITY;
+      const float m_new = fmaxf(m_own[r], GroupMax16(sc));
+      const float shift = m_new == -INFINITY ? 0.0f : m_new;
+      const float p = __builtin_amdgcn_exp2f(sc - shift);
+      const float alpha = __builtin_amdgcn_exp2f(m_own[r] - shift);
+      l_own[r] = fmaf(l_own[r], alpha, p);
+      m_own[r] = m_new;
+      moved = moved || alpha != 1.0f;
+      const int h = HPL * kg + r;
+      if (G >= 4 || h < G) {
+        s_p[wave][n][h] = p;
+        if (n == 0)
           s_alpha[wave][h] = alpha;
       }
     }
     WaveSync();
-    // P V: lane owns dimensions 8 dg .. + 7 of every head of the group.
+    // P V: lane owns dimensions 8 dg .. + 7 of every head of the group. The
+    // rescale by exactly 1 (no head's maximum moved) is skipped.
+    if (__ballot(moved)) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float al = s_alpha[wave][h];
+      for (int h = 0; h < G; ++h) {
+        const float al = s_alpha[wave][h];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        acc[h][i] *= al;
+        for (int i = 0; i < 8; ++i)
+          acc[h][i] *= al;
+      }
     }
 #pragma unroll
     for (int i = 0; i < KPL; ++i) {
       const int o = kq + KG * i;
-      float vf[8];
       const unsigned w4[4] = {vr[i].x, vr[i].y, vr[i].z, vr[i].w};
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        vf[2 * d] = HalfBitsToFloat(w4[d] & 0xffffu);
-        vf[2 * d + 1] = HalfBitsToFloat(w4[d] >> 16);
-      }
 #pragma unroll
       for (int h = 0; h < G; ++h) {
         const float p = s_p[wave][o][h];
+        // acc += p v with the F16 v read as an exact FP32 value.
 #pragma unroll
-        for (int d = 0; d < 8; ++d)
-          acc[h][d] = fmaf(p, vf[d], acc[h][d]);
+        for (int d = 0; d < 4; ++d) {
+          asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,0,0] op_sel_hi:[0,1,0]"
+              : "+v"(acc[h][2 * d]) : "v"(p), "v"(w4[d]));
+          asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[0,1,0] op_sel_hi:[0,1,0]"
+              : "+v"(acc[h][2 * d + 1]) : "v"(p), "v"(w4[d]));
+        }
       }
     }
-    WaveSync();  // the next group rewrites s_tile, s_p and s_alpha
-#pragma unroll
-    for (int s2 = 0; s2 < S; ++s2)
-      kr[s2] = kn[s2];
-#pragma unroll
-    for (int i = 0; i < KPL; ++i)
-      vr[i] = vn[i];
+    WaveSync();  // the next group rewrites s_p and s_alpha
+  };
+  // Two register sets in turn: each group's loads are in flight while the
+  // group before it is computed (past the span: zeros, no traffic).
+  uint4 kn[S], vn[KPL];
+  for (int j = wave; j < ngroups; j += 2 * NW) {
+    fetch(j + NW, kn, vn);
+    step(j, kr, vr);
+    if (j + NW >= ngroups)
+      break;
+    fetch(j + 2 * NW, kr, vr);
+    step(j + NW, kn, vn);
   }
 
   // Merge the key quarters (eighths for D = 64) across lanes, then the
@@ -494,11 +527,12 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
     }
   }
 #pragma unroll
-  for (int r = 0; r < PAIRS; ++r) {
-    const int idx = lane + 64 * r, h = idx >> 4;
-    if (h < G && (idx & 15) == 0) {
+  for (int r = 0; r < HPL; ++r) {
+    const int h = HPL * kg + r;
+    const float l = GroupSum16(l_own[r]);
+    if (h < G && n == 0) {
       s_m[wave][h] = m_own[r];
-      s_l[wave][h] = l_own[r];
+      s_l[wave][h] = l;
     }
   }
   __syncthreads();
@@ -512,12 +546,20 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
 #pragma unroll
     for (int w = 0; w < NW; ++w)
       top = fmaxf(top, s_m[w][h]);
+    if (held)
+      top = fmaxf(top, s_m[NW][h]);
     float l = 0.0f, av = 0.0f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      const float wt = s_m[w][h] == -INFINITY ? 0.0f : expf(s_m[w][h] - top);
+      const float wt = s_m[w][h] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s_m[w][h] - top);
       l = fmaf(s_l[w][h], wt, l);
       av = fmaf(s_acc[w][h][d], wt, av);
+    }
+    if (held) {
+      const float wt =
+          s_m[NW][h] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(s_m[NW][h] - top);
+      l += wt;
+      av = fmaf(HalfBitsToFloat(s_kv[1][d]), wt, av);
     }
     const int head = g * G + h;
     if (unmerged) {
@@ -536,7 +578,7 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
   if constexpr (NW == kAttnWaves) {
     if (split) {  // uniform over the block
       __shared__ int s_last;
-      __shared__ float s_w[kMaxParts][G], s_lv[kMaxParts][G], s_top[G], s_den[G];
+      __shared__ float s_w[kMaxParts][G], s_lv[kMaxParts][G], s_den[G];
       // Every thread's partial stores have completed before the arrival.
       // The hand-over is relaxed on purpose, and is ordered by how gfx950
       // carries out agent-scope accesses rather than by C++ release /
@@ -565,7 +607,7 @@ __launch_bounds__(NW * 64) __global__ void DecodeAttentionKernel(
       __syncthreads();
       if (s_last)
         MergeSpans<D, G, NW * 64>(item, g, kv_heads, partial, s_gate, out, ldo, s_w, s_lv,
-                                  s_top, s_den);
+                                  s_den);
     }
   }
 }

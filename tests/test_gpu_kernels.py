@@ -684,3 +684,52 @@ def test_projection_conv_image(H, B):
         # the shifted part of the window is copied, not recomputed
         keep = hist[r].reshape(H, Lw - 1)[:, 1:]
         assert np.array_equal(h2.reshape(H, Lw - 1)[:, :-1], keep)
+
+
+@pytest.mark.parametrize("heads,kv,D", [(8, 4, 64), (16, 4, 128), (16, 2, 128)])
+@pytest.mark.parametrize("window", [0, 5, 200])
+def test_fused_attention_group_and_ring_edges(heads, kv, D, window):
+    """The fused launch at the edges of its 16-key groups and of its rings:
+    rows whose only key is the current one, spans a key short of, at and past
+    whole groups, rings under 16 slots, exactly full and odd sized ones whose
+    groups wrap; against the oracle's step, with the gate of the ragged test."""
+    from test_oracle import powf
+    n, theta, stride = 8, 1e4, kv * D
+    positions = [0, 1, 15, 16, 17, 63, 64, 65] if not window else \
+        [0, window - 1, window, 3 * window + 7, 1000, 1023, 40, 16]
+    caps = [p + 1 for p in positions] if not window else \
+        [window + e for e in (0, 0, 1, 0, 3, 16, 11, 59)]
+    tag = f"age.{heads}.{kv}.{D}.{window}"
+    ld = (heads + 2 * kv) * D + heads + 4
+    qkv = L.normal(SEED, tag, n * ld).reshape(n, ld)
+    k_off, v_off, g_off = heads * D, (heads + kv) * D, (heads + 2 * kv) * D
+    qn, kn = L.normal(SEED, tag + "q", D, 1, 0.02), L.normal(SEED, tag + "k", D, 1, 0.02)
+    rk = [L.half_normal(SEED, f"{tag}.rk{r}", caps[r] * stride) for r in range(n)]
+    rv = [L.half_normal(SEED, f"{tag}.rv{r}", caps[r] * stride) for r in range(n)]
+    dk, dv = [L.DeviceBuffer.of(b) for b in rk], [L.DeviceBuffer.of(b) for b in rv]
+    tk, tv = pointer_table([b.addr for b in dk]), pointer_table([b.addr for b in dv])
+    pos = np.array(positions, np.uint32)
+    dpos, dcap = L.DeviceBuffer.of(pos), L.DeviceBuffer.of(np.array(caps, np.uint32))
+    freq = powf(theta, np.float32(-2.0) * np.arange(D // 2, dtype=np.float32) / np.float32(D))
+    dfreq, dqn, dkn, dq = (L.DeviceBuffer.of(t) for t in (freq, qn, kn, qkv))
+    items = (L.AttentionItem * 64)()
+    count = L.check(L.lib().lfm3_attention_plan(L.ptr(pos), n, window, items, 64))
+    ditems = L.DeviceBuffer.of(np.frombuffer(items, np.uint8, count * C_ITEM).copy())
+    ws_bytes = L.lib().lfm3_attention_workspace_bytes(count, n, heads, kv, D)
+    ws = L.DeviceBuffer.of(np.zeros(ws_bytes, np.uint8))
+    dout = L.DeviceBuffer(n * heads * D * 4)
+    L.check(L.lib().lfm3_decode_heads_attention_ragged(
+        dq.addr, dq.addr + 4 * k_off, dq.addr + 4 * v_off, ld, dq.addr + 4 * g_off, ld, dqn.addr,
+        dkn.addr, dfreq.addr, None, tk.addr, tv.addr, dpos.addr, dcap.addr, ditems.addr, count,
+        dout.addr, heads * D, n, heads, kv, D, 1e-5, ws.addr, ws_bytes, None))
+    L.synchronize()
+    out = dout.download(np.float32, n * heads * D).reshape(n, heads * D)
+    for r in range(n):
+        want, _, _ = O.attention_step(qkv[r, :k_off], qkv[r, k_off:v_off], qkv[r, v_off:g_off],
+                                      qkv[r, g_off:g_off + heads], qn, kn,
+                                      None if window else np.ones(D // 2, np.float32),
+                                      O.half_to_float(rk[r]), O.half_to_float(rv[r]), heads, kv,
+                                      D, positions[r], caps[r], window, theta, bool(window), 1e-5,
+                                      True)
+        ok, err = within(out[r], want)
+        assert ok, (r, err)
