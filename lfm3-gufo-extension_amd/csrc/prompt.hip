@@ -20,6 +20,7 @@
 // parts in part order, so no launch merges blocks through memory.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -50,20 +51,20 @@ constexpr int kGemmRT = 4, kGemmTT = 4, kGemmStages = 3;
 // stages and a KG-th of the block's chunks; the groups' sums meet in LDS
 // and add in group order.
 template<int WR, int WT, bool kHalf = false, int kStageCount = kGemmStages, int TT = kGemmTT,
-         int KG = 1>
+         int KG = 1, int RT = kGemmRT>
 struct GemmShape {
-  static constexpr int kWR = WR, kWT = WT, kTT = TT, kKG = KG;
+  static constexpr int kWR = WR, kWT = WT, kTT = TT, kKG = KG, kRT = RT;
   static constexpr bool kHalfTiles = kHalf;
   static constexpr int kStages = kStageCount;  // LDS pipeline stages: 2 or 3
   static constexpr int kWaves = WR * WT;       // waves of a K group
   static constexpr int kThreads = 64 * kWaves * KG;
-  static constexpr int kTiles = WR * kGemmRT;  // weight tiles a block
+  static constexpr int kTiles = WR * RT;  // weight tiles a block
   static constexpr int kTokens = WT * TT * 16;
   static constexpr int kTileW = kHalf ? 2 * kTileCodeBytes : kTileCodeBytes;
   static constexpr int kW = kTokens * 128;
   static constexpr int kS = kW + kTiles * kTileW;
-  static constexpr int kBytes = kS + kTiles * kTileScales * 2;  // a group's stage
-  static constexpr int kSums = (KG - 1) * kWaves * kGemmRT * TT * 64 * 16;
+  static constexpr int kBytes = kS + WR * 4 * kTileScales * 2;  // a group's stage
+  static constexpr int kSums = (KG - 1) * kWaves * RT * TT * 64 * 16;
   static_assert(kSums <= KG * kBytes, "the groups' sums fit the first stage array");
   // Row maxima of 128 outputs come from the block that owns their 16 tiles.
   static constexpr bool kMaxima = kTiles == 16 && KG == 1;
@@ -88,6 +89,10 @@ template<bool kHalf>
 using Rows64Tokens128 = GemmShape<1, 4, kHalf, kGemmStages, 2, 2>;
 template<bool kHalf>
 using Rows128Tokens64 = GemmShape<2, 2, kHalf, kGemmStages, 2, 2>;
+// 96 weight rows (three tiles a wave): where 128 leave a quarter of the CUs
+// idle (6144 x 2048 at 512 rows: 192 blocks, 27.8 us; 256 of these, 24.6).
+// The FP16 tiles only: on code tiles the 128-row block gives the same sums.
+using Rows96Shape = GemmShape<2, 4, true, kGemmStages, 2, 1, 3>;
 // The same 256 x 128 block tile on FP16 tiles in 16 waves of 64 rows x 32
 // tokens: four waves a SIMD instead of two hide more of the LDS and MFMA
 // latency, for half again the LDS operand reads a MFMA (the SwiGLU GEMM
@@ -383,16 +388,17 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
                              int row_blocks, int token_blocks, int parts,
                              std::size_t part_stride,
                              unsigned* __restrict__ row_max, const HiddenHalves tail) {
-  constexpr int RT = kGemmRT, TT = Shape::kTT;
+  constexpr int RT = Shape::kRT, TT = Shape::kTT;
   using Stage = Shape;
   constexpr int KG = Shape::kKG, kGroupThreads = 64 * Shape::kWaves;
   constexpr int A_LOADS = Shape::kTokens * 8 / kGroupThreads;  // 16-byte loads a lane
-  constexpr int W_LOADS = Shape::kTiles / Shape::kWaves;         // tiles a wave loads
   constexpr int kTileW = Shape::kTileW;                           // bytes of a tile's chunk
   constexpr int W_PIECES = kTileW / kTileCodeBytes;               // 1 KB loads a tile
+  // 1 KB loads of a wave: consecutive ones, the first W_MORE waves one more.
+  constexpr int W_UNITS = Shape::kTiles * W_PIECES;
+  constexpr int W_LOADS = W_UNITS / Shape::kWaves, W_MORE = W_UNITS % Shape::kWaves;
   static_assert(A_LOADS * kGroupThreads == Shape::kTokens * 8, "A loads cover the rows");
-  static_assert(W_LOADS * Shape::kWaves == Shape::kTiles, "W loads cover the tiles");
-  static_assert(RT == 4 && Shape::kWR <= Shape::kWaves, "scale groups of four tiles");
+  static_assert(RT <= 4 && Shape::kWR <= Shape::kWaves, "scale groups of four tiles");
   // One array per stage (not one indexed by stage) lets the compiler see
   // that a stage's reads never alias the other stages' loads in flight.
   __shared__ __attribute__((aligned(16))) std::uint8_t s_st0[KG * Stage::kBytes];
@@ -444,17 +450,21 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
     const int seg = (lane & 7) ^ (t & 7);
     a_off[j] = (unsigned(min(t, n - 1 - tok0)) * unsigned(lda) + unsigned(seg * 8)) * 2u;
   }
-  unsigned w_tile[W_LOADS];  // byte offset of each loaded tile's chunk 0 (uniform)
+  constexpr int W_SLOTS = W_LOADS + (W_MORE ? 1 : 0);
+  const bool loads_more = W_MORE && wave < W_MORE;
+  const int w_first = wave * W_LOADS + (W_MORE ? min(wave, W_MORE) : 0);
+  unsigned w_unit[W_SLOTS];  // byte offset of each load in its tile's chunk 0 (uniform)
 #pragma unroll
-  for (int j = 0; j < W_LOADS; ++j)
-    w_tile[j] = unsigned(min(btile0 + wave * W_LOADS + j, row_tiles - 1)) *
-                unsigned(nchunks * kTileW);
+  for (int j = 0; j < W_SLOTS; ++j)
+    w_unit[j] = unsigned(min(btile0 + (w_first + j) / W_PIECES, row_tiles - 1)) *
+                    unsigned(nchunks * kTileW) +
+                unsigned((w_first + j) % W_PIECES * kTileCodeBytes);
   const unsigned w_off = unsigned(lane) * 16u;
-  // Scales: wave g < Shape::kWR loads group g; lane L brings tile 4 g + L % 4's
+  // Scales: wave g < Shape::kWR loads group g; lane L brings tile RT g + L % 4's
   // dword L / 4 (row L / 4's two block scales).
   const bool loads_scales = wave < Shape::kWR;
   const unsigned s_off =
-      unsigned(min(btile0 + wave * 4 + (lane & 3), row_tiles - 1)) *
+      unsigned(min(btile0 + wave * RT + min(lane & 3, RT - 1), row_tiles - 1)) *
           unsigned(nchunks * kTileScales * 2) +
       unsigned((lane >> 2) * 4);
   const auto issue = [&](int c, std::uint8_t* stages) {
@@ -464,21 +474,26 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
       BufferToLds16(a_res, a_off[j], unsigned(c * kChunk * 2),
                     stage + (wave * A_LOADS + j) * 1024);
 #pragma unroll
-    for (int j = 0; j < W_LOADS; ++j)
-#pragma unroll
-      for (int piece = 0; piece < W_PIECES; ++piece)
-        BufferToLds16(w_res, w_off, w_tile[j] + unsigned(c * kTileW + piece * kTileCodeBytes),
-                      stage + Stage::kW + (wave * W_LOADS + j) * kTileW + piece * kTileCodeBytes);
+    for (int j = 0; j < W_SLOTS; ++j)
+      if (j < W_LOADS || loads_more)
+        BufferToLds16(w_res, w_off, w_unit[j] + unsigned(c * kTileW),
+                      stage + Stage::kW + (w_first + j) * kTileCodeBytes);
     if (loads_scales)
       BufferToLds4(s_res, s_off, unsigned(c * kTileScales * 2),
                    stage + Stage::kS + wave * 4 * kTileScales * 2);
   };
   // Waits until at most one chunk's loads of this wave remain in flight.
   const auto wait_all_but_one_chunk = [&]() {
-    if (loads_scales)
-      __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS * W_PIECES + 1));
-    else
-      __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS * W_PIECES));
+    if (W_MORE && loads_more) {
+      if (loads_scales)
+        __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS + 2));
+      else
+        __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS + 1));
+    } else if (loads_scales) {
+      __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS + 1));
+    } else {
+      __builtin_amdgcn_s_waitcnt(WaitVm(A_LOADS + W_LOADS));
+    }
   };
 
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -556,7 +571,7 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
     }
     __builtin_amdgcn_sched_barrier(0);
     const uint4 sc4 = *reinterpret_cast<const uint4*>(
-        stage + Stage::kS + wr * RT * kTileScales * 2 + (lane & 15) * 16);
+        stage + Stage::kS + wr * 4 * kTileScales * 2 + (lane & 15) * 16);
     sc[0] = sc4.x;
     sc[1] = sc4.y;
     sc[2] = sc4.z;
@@ -864,17 +879,19 @@ __global__ void SumPartsKernel(float* __restrict__ y, std::size_t part_stride, i
 // of those 130 launches (where two blocks would share a CU, at most 25%).
 struct ShapeCost {
   int tokens, tiles, groups;
+  bool pairs;  // a wave's tiles come in gate/up pairs
   float round, step, fill;
 };
 template<class Shape>
 constexpr ShapeCost CostOf(float round, float step, float fill) {
-  return {Shape::kTokens, Shape::kTiles, Shape::kKG, round, step, fill};
+  return {Shape::kTokens, Shape::kTiles, Shape::kKG, Shape::kRT % 2 == 0, round, step, fill};
 }
 constexpr ShapeCost kShapeCosts[] = {
     CostOf<Rows64Tokens32<true>>(1.55f, 0.758f, 0.083f),
     CostOf<Rows64Tokens64<true>>(1.91f, 0.680f, 0.215f),
     CostOf<Rows64Tokens128<true>>(3.11f, 0.648f, 0.224f),
     CostOf<Rows128Tokens64<true>>(3.22f, 0.708f, 0.234f),
+    CostOf<Rows96Shape>(2.20f, 0.466f, 0.207f),
     CostOf<NarrowHalfShape>(3.28f, 0.558f, 0.232f),
     CostOf<WideHalfShape>(5.52f, 0.872f, 0.435f),
 };
@@ -908,8 +925,10 @@ int BestShape(int row_tiles, int tokens, int nchunks, int parts, bool swiglu) {
   float least = LaunchCost(kShapeCosts[kWide], row_tiles, tokens, nchunks, parts);
   for (int i = 0; i < kWide; ++i) {
     const float cost = LaunchCost(kShapeCosts[i], row_tiles, tokens, nchunks, parts);
-    if (cost < least && (!swiglu || std::size_t(ShapeBlocks(kShapeCosts[i], row_tiles, tokens)) <=
-                                        SwiGLUFlags(row_tiles, std::uint32_t(tokens)))) {
+    const bool takes = !swiglu || (kShapeCosts[i].pairs &&
+                                   std::size_t(ShapeBlocks(kShapeCosts[i], row_tiles, tokens)) <=
+                                       SwiGLUFlags(row_tiles, std::uint32_t(tokens)));
+    if (cost < least && takes) {
       best = i;
       least = cost;
     }
@@ -1009,9 +1028,11 @@ auto Launcher(int i, bool half) {
   constexpr decltype(&LaunchGemm<kSwiGLU, WideShape>) kLaunchers[2][kShapes] = {
       {LaunchGemm<kSwiGLU, Rows64Tokens32<false>>, LaunchGemm<kSwiGLU, Rows64Tokens64<false>>,
        LaunchGemm<kSwiGLU, Rows64Tokens128<false>>, LaunchGemm<kSwiGLU, Rows128Tokens64<false>>,
-       LaunchGemm<kSwiGLU, NarrowShape>, LaunchGemm<kSwiGLU, WideShape>},
+       LaunchGemm<kSwiGLU, NarrowShape>, LaunchGemm<kSwiGLU, NarrowShape>,
+       LaunchGemm<kSwiGLU, WideShape>},
       {LaunchGemm<kSwiGLU, Rows64Tokens32<true>>, LaunchGemm<kSwiGLU, Rows64Tokens64<true>>,
        LaunchGemm<kSwiGLU, Rows64Tokens128<true>>, LaunchGemm<kSwiGLU, Rows128Tokens64<true>>,
+       LaunchGemm<kSwiGLU, std::conditional_t<kSwiGLU, NarrowHalfShape, Rows96Shape>>,
        LaunchGemm<kSwiGLU, NarrowHalfShape>, LaunchGemm<kSwiGLU, WideHalfShape>}};
   return kLaunchers[half][i];
 }

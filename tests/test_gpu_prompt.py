@@ -186,7 +186,9 @@ def test_gemm_half_tiles_identical(M, K, n, parts, swiglu):
     (6144, 448, 64, 1),    # 64 x 64 blocks: seven chunks over three K groups
     (6144, 448, 65, 2),    # 64 x 128 blocks, the second half nearly empty
     (6144, 2048, 300, 1),  # 128 x 64 blocks
-    (6144, 2048, 385, 1),  # 128 x 128 blocks, one row in the last
+    (6144, 2048, 385, 1),  # 96 x 128 blocks, one row in the last
+    (6000, 256, 400, 1),   # 96 x 128 blocks, half a block of weight rows at the end
+    (2048, 2112, 385, 4),  # 128 x 128 blocks, 33 chunks in four parts
     (16, 7680, 17, 8),     # one weight tile
 ])
 def test_gemm_block_shapes(M, K, n, parts):
