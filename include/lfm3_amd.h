@@ -596,8 +596,9 @@ int lfm3_store_kv(const uint16_t* k16, const uint16_t* v16, uint16_t* cache_k,
    round of blocks on the CUs takes, at most 16) keep partial sums, rows x
    heads x (dim + 2) floats a span; this bounds any head grouping and
    serves every call of fewer rows. 0 when the keys fit one span or window
-   > 0. A smaller workspace makes fewer spans; spans of at least 1024 keys
-   have to fit. */
+   > 0. A smaller workspace gives the same output from fewer, longer blocks;
+   as many partial sums as spans of at least 1024 keys would keep have to
+   fit (none for up to 1984 keys). */
 size_t lfm3_prompt_attention_workspace_bytes(uint32_t rows, uint32_t heads,
                                              uint32_t dim, uint32_t position,
                                              uint32_t window);
@@ -625,8 +626,7 @@ int lfm3_prompt_attention(const float* q, uint32_t ldq, const uint16_t* k,
 /* lfm3_prompt_attention with its output written as the output projection's
    FP16 row-scaled activations: row r's heads * dim outputs (the same FP32
    values) go to out + r * lda as fp16(out 2^e) with scale[r] = 2^-e, e =
-   14 - ilogb(max |row|) (lfm3_half_rows of the FP32 output, bit for bit
-   where both calls have the workspaces their functions give).
+   14 - ilogb(max |row|) (lfm3_half_rows of the FP32 output, bit for bit).
    Every call keeps per-span partial sums in the workspace
    (lfm3_prompt_attention_half_workspace_bytes, at least one span); a
    per-row merge writes the rows. lda % 64 == 0, lda >= heads * dim.

@@ -30,6 +30,9 @@
 // at least 256 keys and at most 16 spans; the reference's PromptSplits
 // instead fixes spans of at least 2048 keys, at most 8). Each span stores
 // its maximum, sum and unnormalized output, merged by CombineSpansKernel.
+// Where the workspace holds fewer records than spans, a block walks a group
+// of spans and folds them itself, with the merge's own expressions: the
+// result depends on the call's sizes, never on its workspace.
 #include <algorithm>
 #include <cmath>
 
@@ -58,12 +61,64 @@ int TileSpans(int tiles) {
   return tiles < kSplitTiles ? 1 : std::min(kMaxSpans, tiles / kSpanFloorTiles);
 }
 
-int SpanPlan(int keys, int blocks_per_span, int fill, int room, int& span_keys) {
+int SpanPlan(int keys, int blocks_per_span, int fill, int& span_keys) {
   const int tiles = (keys + kPAKeys - 1) / kPAKeys;
-  const int spans = std::max(
-      1, std::min({fill / std::max(blocks_per_span, 1), TileSpans(tiles), room}));
+  const int spans =
+      std::max(1, std::min(fill / std::max(blocks_per_span, 1), TileSpans(tiles)));
   span_keys = (tiles + spans - 1) / spans * kPAKeys;
   return (keys + span_keys - 1) / span_keys;
+}
+
+// A span's record (maximum m, sum l, output a) folded into a group's: one
+// step of the same expressions whether a block folds the spans that it walks
+// or the merge folds their records. An empty group is (-inf, 0, 0).
+struct SpanFold {
+  float old_weight, new_weight;
+};
+__device__ __forceinline__ SpanFold FoldWeights(float& group_m, float& group_l, float m, float l) {
+  const float top = fmaxf(group_m, m), shift = top == -INFINITY ? 0.0f : top;
+  const SpanFold f{__builtin_amdgcn_exp2f(group_m - shift), __builtin_amdgcn_exp2f(m - shift)};
+  group_m = top;
+  group_l = fmaf(group_l, f.old_weight, l * f.new_weight);
+  return f;
+}
+__device__ __forceinline__ float FoldOutput(float group_a, float a, SpanFold f) {
+  return fmaf(group_a, f.old_weight, a * f.new_weight);
+}
+
+// The last span of its group of `per`.
+__device__ __forceinline__ bool EndsGroup(int s, int splits, int per) {
+  return (s + 1) % per == 0 || s + 1 == splits;
+}
+
+// Spans' records (S of them live) into their groups': a group's record takes
+// the place of its last span's. D outputs a record.
+template<int D>
+__device__ __forceinline__ void FoldGroups(float (&m)[kMaxSpans], float (&l)[kMaxSpans],
+                                           float (&a)[kMaxSpans][D], int splits, int per) {
+  float group_m = -INFINITY, group_l = 0.0f, group_a[D] = {};
+#pragma unroll
+  for (int s = 0; s < kMaxSpans; ++s) {
+    if (s >= splits)
+      break;
+    const SpanFold f = FoldWeights(group_m, group_l, m[s], l[s]);
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+      group_a[i] = FoldOutput(group_a[i], a[s][i], f);
+    if (EndsGroup(s, splits, per)) {
+      m[s] = group_m;
+      l[s] = group_l;
+      group_m = -INFINITY;
+      group_l = 0.0f;
+#pragma unroll
+      for (int i = 0; i < D; ++i) {
+        a[s][i] = group_a[i];
+        group_a[i] = 0.0f;
+      }
+    } else {
+      m[s] = -INFINITY;  // counted in the group's
+    }
+  }
 }
 
 // Keys visible to a query at absolute position p, clipped to a span
@@ -104,13 +159,15 @@ __device__ __forceinline__ void PromptBlock(int b, int row_blocks, int& rb, int&
   pair = xcd + 8 * (i / row_blocks);
 }
 
-template<int D, int G, int CT>
+// kFold: the block's keys (`span` of them) are several of the plan's spans,
+// of `sub` keys each, folded in order as their records are in the merge.
+template<int D, int G, int CT, bool kFold>
 __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
     const float* __restrict__ q, int ldq, const Half* __restrict__ k,
     const Half* __restrict__ v, const float* __restrict__ gate, int ldg,
     const Half* __restrict__ ck, const Half* __restrict__ cv, float* __restrict__ out,
     int ldo, float* __restrict__ partial, int n, int heads, int kv_heads, int position,
-    int capacity, int window, int span, int row_blocks, int splits) {
+    int capacity, int window, int span, int sub, int row_blocks, int splits) {
   static_assert(D == 64 || D == 128, "head dimension");
   constexpr int kCols = 16 * CT * kPAWaves;  // (row, head) columns a block
   static_assert(kCols % G == 0 && G >= 2 && G <= 8, "query group");
@@ -383,6 +440,37 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
     }
   };
 
+  // The open span's state into the group's.
+  f4 group_acc[kFold ? CT : 1][kFold ? kDimBlocks : 1];
+  float group_max[kFold ? CT : 1], group_sum[kFold ? CT : 1];
+  int next_span = span_lo + sub;
+  if constexpr (kFold)
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+#pragma unroll
+      for (int m = 0; m < kDimBlocks; ++m)
+        group_acc[ct][m] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      group_max[ct] = -INFINITY;
+      group_sum[ct] = 0.0f;
+    }
+  const auto close_span = [&]() {
+    if constexpr (kFold)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        const SpanFold f = FoldWeights(group_max[ct], group_sum[ct], maximum[ct],
+                                       SumXor32(SumXor16(sum[ct])));
+#pragma unroll
+        for (int m = 0; m < kDimBlocks; ++m)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            group_acc[ct][m][i] = FoldOutput(group_acc[ct][m][i], acc[ct][m][i], f);
+            acc[ct][m][i] = 0.0f;
+          }
+        maximum[ct] = -INFINITY;
+        sum[ct] = 0.0f;
+      }
+  };
+
   // Tiles: write the prefetched tile to its stage, one barrier (the tile is
   // visible, and every wave is done with the stage written two tiles ago),
   // prefetch the next tile, multiply.
@@ -395,14 +483,32 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
     __syncthreads();
     if (base + kPAKeys <= walk.hi)
       load(base + kPAKeys);
+    if (kFold && base == next_span) {
+      close_span();
+      next_span += sub;
+    }
     if (!wave_live || base > reach.hi || base + kPAKeys <= reach.lo)
       continue;
     compute(st, base);
   }
 
+  if constexpr (kFold) {
+    // The last walked span, and those of the group past the block's rows:
+    // empty records, which the merge would add too.
+    close_span();
+    for (; next_span <= span_hi && next_span < position + n; next_span += sub)
+      close_span();
+  }
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
-    const float total = SumXor32(SumXor16(sum[ct]));
+    float total = SumXor32(SumXor16(sum[ct]));
+    if constexpr (kFold) {
+      total = group_sum[ct];
+      maximum[ct] = group_max[ct];
+#pragma unroll
+      for (int m = 0; m < kDimBlocks; ++m)
+        acc[ct][m] = group_acc[ct][m];
+    }
     if (!live[ct])
       continue;
     // Lane L holds dimensions 16 m + 4 (L / 16) + i of its column.
@@ -433,26 +539,29 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
 }
 
 // hip/ops.hip:1692-1709: merges key spans (base-2 maxima); one block per
-// (row, head), one thread per dimension.
+// (row, head), one thread per dimension. The spans of a group of `per` fold
+// in order, then the groups add against their common maximum.
 template<int D>
 __launch_bounds__(D) __global__
     void CombineSpansKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                             int ldg, float* __restrict__ out, int ldo, int n, int heads,
-                            int splits) {
+                            int splits, int per) {
   const int rh = blockIdx.x, d = threadIdx.x;
   const int row = rh / heads, head = rh % heads;
   const std::size_t rows = std::size_t(n) * heads;
   // Every load (each span's maximum, sum and output element, and the gate)
   // is issued before any arithmetic: one memory round trip.
-  float m[kMaxSpans], l[kMaxSpans], a[kMaxSpans];
+  float m[kMaxSpans], l[kMaxSpans], a[kMaxSpans][1];
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s) {
     const float* part = partial + (s * rows + rh) * (D + 2);
     m[s] = s < splits ? part[0] : -INFINITY;
     l[s] = s < splits ? part[1] : 0.0f;
-    a[s] = s < splits ? part[2 + d] : 0.0f;
+    a[s][0] = s < splits ? part[2 + d] : 0.0f;
   }
   const float g = gate[std::size_t(row) * ldg + head];
+  if (per > 1)
+    FoldGroups(m, l, a, splits, per);
   float maximum = -INFINITY;
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s)
@@ -460,10 +569,10 @@ __launch_bounds__(D) __global__
   float sum = 0.0f, acc = 0.0f;
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s) {
-    if (s < splits) {
+    if (s < splits && EndsGroup(s, splits, per)) {
       const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
       sum = fmaf(l[s], w, sum);
-      acc = fmaf(a[s], w, acc);
+      acc = fmaf(a[s][0], w, acc);
     }
   }
   out[std::size_t(row) * ldo + head * D + d] = (acc / sum) / (1.0f + expf(-g));
@@ -482,7 +591,8 @@ template<int D>
 __launch_bounds__(1024) __global__
     void CombineRowsHalfKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                                int ldg, Half* __restrict__ out, int lda,
-                               float* __restrict__ scale, int n, int heads, int splits) {
+                               float* __restrict__ scale, int n, int heads, int splits,
+                               int per) {
   __shared__ float s_max[16];
   const int row = blockIdx.x, tid = threadIdx.x;
   constexpr int kPerHead = D / kCombineDims;
@@ -506,6 +616,8 @@ __launch_bounds__(1024) __global__
     a[s][3] = v1.y;
   }
   const float g = live ? gate[std::size_t(row) * ldg + head] : 0.0f;
+  if (per > 1)
+    FoldGroups(m, l, a, splits, per);
   float maximum = -INFINITY;
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s)
@@ -513,7 +625,7 @@ __launch_bounds__(1024) __global__
   float sum = 0.0f, acc[kCombineDims] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s) {
-    if (s < splits) {
+    if (s < splits && EndsGroup(s, splits, per)) {
       const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
       sum = fmaf(l[s], w, sum);
 #pragma unroll
@@ -555,7 +667,11 @@ struct PromptArgs {
   float* out;
   int ldo;
   float* partial;
-  int n, heads, kv_heads, position, capacity, window, span, splits;
+  int n, heads, kv_heads, position, capacity, window;
+  // Keys of a planned span; records the launch writes; planned spans a group,
+  // and whether a block walks a group (else one span).
+  int span, splits, per;
+  bool fold;
   // FP16 rows out (partials for every span, merged by CombineRowsHalfKernel).
   Half* out16 = nullptr;
   int lda = 0;
@@ -569,11 +685,9 @@ int ColumnTiles(int position, int n, int window, int group) {
   return window == 0 && position + n > 4096 && n * group > 16 * kPAWaves ? 2 : 1;
 }
 
-// The span plan of one call: span length and count for the tile launch of
-// the chosen shape (spans > 1 only for a history without a window), at most
-// `room` spans where the workspace holds no more.
-int PlanCall(int n, int position, int window, int group, int kv_heads, int dim, int room,
-             int& span) {
+// The planned spans of one call and their length (more than one only for a
+// history without a window).
+int PlanSpans(int n, int position, int window, int group, int kv_heads, int dim, int& span) {
   const int keys = position + n;
   span = keys;
   if (window)
@@ -584,15 +698,16 @@ int PlanCall(int n, int position, int window, int group, int kv_heads, int dim, 
   // Blocks a round: two a CU where 64 dimensions and one column tile leave
   // the registers (300 rows after 3000 of 32 x 64 heads 69.6 us against 71.4).
   const int fill = dim == 64 && column_tiles == 1 ? 512 : 256;
-  const int spans = SpanPlan(keys, blocks_per_span, fill, room, span);
+  const int spans = SpanPlan(keys, blocks_per_span, fill, span);
   if (spans == 1)
     span = keys;
   return spans;
 }
 
-// Spans that a call's workspace has to hold: spans of at least 1024 keys, at
-// most 16, for about one block a CU of the larger block. A workspace between
-// this and the plan's own need takes fewer spans.
+// Records that a call's workspace has to hold: one for each span of at least
+// 1024 keys, at most 16, for about one block a CU of the larger block. The
+// planned spans form as many groups (at most), so that a workspace between
+// this and the plan's own need serves with a block a group.
 int LeastSpans(int n, int position, int window, int group, int kv_heads) {
   if (window)
     return 1;
@@ -603,33 +718,35 @@ int LeastSpans(int n, int position, int window, int group, int kv_heads) {
   return (tiles + span_tiles - 1) / span_tiles;
 }
 
-template<int D, int G, int CT>
+template<int D, int G, int CT, bool kFold>
 void LaunchTiles(const PromptArgs& a, hipStream_t s) {
   constexpr int kRows = 16 * CT * kPAWaves / G;
   const int row_blocks = (a.n + kRows - 1) / kRows;
-  // 8 XCD slots of row_blocks blocks per group of 8 (span, KV head) pairs.
+  // 8 XCD slots of row_blocks blocks per group of 8 (record, KV head) pairs.
   const int pairs = a.splits * a.kv_heads;
   const int blocks = (pairs + 7) / 8 * 8 * row_blocks;
-  PromptAttentionKernel<D, G, CT><<<blocks, kPAThreads, 0, s>>>(
+  PromptAttentionKernel<D, G, CT, kFold><<<blocks, kPAThreads, 0, s>>>(
       a.q, a.ldq, a.k, a.v, a.gate, a.ldg, a.ck, a.cv, a.out, a.ldo,
       a.splits > 1 || a.out16 ? a.partial : nullptr, a.n, a.heads, a.kv_heads, a.position,
-      a.capacity,
-      a.window, a.span, row_blocks, a.splits);
+      a.capacity, a.window, kFold ? a.per * a.span : a.span, a.span, row_blocks, a.splits);
 }
 
 template<int D, int G>
 void LaunchPrompt(const PromptArgs& a, hipStream_t s) {
-  if (ColumnTiles(a.position, a.n, a.window, G) == 2)
-    LaunchTiles<D, G, 2>(a, s);
+  if (a.fold)  // one column tile: the group's state takes the other's registers
+    LaunchTiles<D, G, 1, true>(a, s);
+  else if (ColumnTiles(a.position, a.n, a.window, G) == 2)
+    LaunchTiles<D, G, 2, false>(a, s);
   else
-    LaunchTiles<D, G, 1>(a, s);
+    LaunchTiles<D, G, 1, false>(a, s);
+  const int per = a.fold ? 1 : a.per;
   if (a.out16) {
     const int threads = (a.heads * (D / kCombineDims) + 63) / 64 * 64;
     CombineRowsHalfKernel<D><<<a.n, threads, 0, s>>>(a.partial, a.gate, a.ldg, a.out16, a.lda,
-                                                     a.scale, a.n, a.heads, a.splits);
+                                                     a.scale, a.n, a.heads, a.splits, per);
   } else if (a.splits > 1) {
     CombineSpansKernel<D><<<a.n * a.heads, D, 0, s>>>(a.partial, a.gate, a.ldg, a.out, a.ldo,
-                                                       a.n, a.heads, a.splits);
+                                                       a.n, a.heads, a.splits, per);
   }
 }
 
@@ -709,10 +826,15 @@ int PromptAttention(const float* q, std::uint32_t ldq, const std::uint16_t* k,
   const std::size_t need = least > 1 || half ? least * span_bytes : 0;
   if (need && (!workspace || workspace_bytes < need))
     return Fail(LFM3_E_INVALID, "LFM3 prompt attention workspace too small");
-  const int room = int(std::min<std::size_t>(workspace ? workspace_bytes / span_bytes : 1,
-                                             kMaxSpans));
-  a.splits = PlanCall(int(rows), int(position), int(window), int(group), int(kv_heads), int(dim),
-                      room, a.span);
+  // The plan depends on the sizes alone; a workspace that holds fewer records
+  // than spans takes a block and a record a group (group <= least, so they
+  // fit; a single group without a workspace writes its rows itself).
+  const std::size_t room = workspace ? workspace_bytes / span_bytes : 0;
+  const int spans = PlanSpans(int(rows), int(position), int(window), int(group), int(kv_heads),
+                              int(dim), a.span);
+  a.per = (spans + least - 1) / least;
+  a.fold = a.per > 1 && std::size_t(spans) > room;
+  a.splits = a.fold ? (spans + a.per - 1) / a.per : spans;
   a.q = q;
   a.ldq = int(ldq);
   a.k = k;

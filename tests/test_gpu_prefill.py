@@ -497,6 +497,61 @@ def test_prompt_attention_span_plans(n, P, H, KH, D):
     assert np.max(np.abs(rows - want)) < 1e-3
 
 
+@pytest.mark.parametrize("n,P,H,KH,D", [
+    (64, 700, 16, 4, 128),     # three spans; no workspace was ever asked for (one group)
+    (300, 3000, 16, 4, 128),   # six spans in three groups
+    (300, 5000, 16, 4, 128),   # two column tiles a wave; twelve spans in groups of three
+    (33, 2500, 8, 4, 128),     # few rows, two groups of five spans
+    (512, 3000, 16, 4, 128),   # four spans in two groups, rows that reach the last span late
+    (200, 6000, 8, 2, 64),     # a last group shorter than the others
+])
+def test_prompt_attention_result_is_the_same_in_every_workspace(n, P, H, KH, D):
+    """The FP32 rows bit for bit the same whatever accepted workspace they
+    are given, none at all where none is asked for, and the FP16 rows their
+    conversion in every pair of workspaces; within the gate of FP64."""
+    tag = f"{n}.{P}.{H}.{D}"
+    stride, cap = KH * D, P + n
+    q = L.normal(SEED, f"pws.q.{tag}", n * H * D).reshape(n, H * D)
+    gates = L.normal(SEED, f"pws.g.{tag}", n * H).reshape(n, H)
+    bits = [L.half_normal(SEED, f"pws.{t}.{tag}", r * stride)
+            for t, r in (("k", n), ("v", n), ("ck", cap), ("cv", cap))]
+    dq, dg = L.DeviceBuffer.of(np.ascontiguousarray(q)), L.DeviceBuffer.of(gates)
+    dk, dv, dck, dcv = (L.DeviceBuffer.of(b) for b in bits)
+    span = n * H * (D + 2) * 4
+    most = L.lib().lfm3_prompt_attention_workspace_bytes(n, H, D, P, 0) // span
+    assert 1 < most <= 16
+    out, rows, refused = {}, {}, set()
+    for records in range(most + 1):
+        ws = L.DeviceBuffer(max(records * span, 4))
+        dy, da = L.DeviceBuffer(n * H * D * 4), L.DeviceBuffer(n * H * D * 2)
+        ds = L.DeviceBuffer(n * 4)
+        args = (dq.addr, H * D, dk.addr, dv.addr, dg.addr, H, dck.addr, dcv.addr)
+        sizes = (n, H, KH, D, P, cap, 0, ws.addr if records else None, records * span, None)
+        if L.lib().lfm3_prompt_attention(*args, dy.addr, H * D, *sizes) == L.E_INVALID:
+            refused.add(records)
+        else:
+            L.synchronize()
+            out[records] = dy.download(np.float32, n * H * D).reshape(n, H * D)
+        if L.lib().lfm3_prompt_attention_half(*args, da.addr, H * D, ds.addr, *sizes) == 0:
+            L.synchronize()
+            rows[records] = (da.download(np.uint16, n * H * D).reshape(n, H * D),
+                             ds.download(np.float32, n))
+    print(f"[prompt attention workspaces] {tag}: refused {sorted(refused)}", flush=True)
+    assert out.keys() | refused == set(range(most + 1)) and most in out and most in rows
+    assert not refused or max(refused) < min(out)
+    want = prompt_attention_fp64(q, gates, *[O.half_to_float(b) for b in bits], n, H, KH, D, P,
+                                 cap, 0)
+    full = out[most]
+    assert np.max(np.abs(full - want)) < 1e-3
+    for got in out.values():
+        assert np.array_equal(got.view(np.uint32), full.view(np.uint32))
+    _, exps = O.half_rows(full)
+    half = O.float_to_half(np.ldexp(full, exps[:, None]).astype(np.float32))
+    for a, scale in rows.values():
+        assert np.array_equal(a, half)
+        assert np.array_equal(scale, np.ldexp(np.float32(1), -exps).astype(np.float32))
+
+
 def test_prompt_attention_workspace_serves_fewer_rows():
     """A workspace sized for some rows and position holds every call of
     fewer, and none is asked for where nothing splits."""
