@@ -242,9 +242,12 @@ int lfm3_q8_gemm_swiglu(const void* codes, const void* scales, uint32_t rows,
    maxima through to memory and then stores `seq` in its flag; a trailing
    block waits for the flags of its token block's GEMM blocks (bounded: a
    timeout stores 1 to *error, which may be NULL, and the block goes on).
-   flags: lfm3_q8_gemm_swiglu_flags_bytes(rows, tokens), zeroed once; seq:
-   nonzero and different from the previous call's on the same flags; calls
-   on the same flags must not overlap. out must not alias a (the GEMM reads
+   flags: lfm3_q8_gemm_swiglu_flags_bytes(rows, tokens), zeroed once; a call
+   leaves `seq` in all of them (how they map to blocks depends on the token
+   count). seq: nonzero and not in any of the call's flags before it: other
+   than the previous call's while that size stays the same (any tokens up to
+   512), else other than every earlier one (a counter; zero the flags again
+   when it wraps). Calls on the same flags must not overlap. out must not alias a (the GEMM reads
    a while trailing blocks write out). rows % 4 == 0 and rows <= 8192, ldy
    % 4 == 0, out_ld % 64 == 0. Replaces: gpu::ProjectFfn's gate/up GEMM
    and the down projection's HalfRowsFromMax (q8_prefill.hpp:53-74;

@@ -249,6 +249,7 @@ struct HiddenHalves {
   unsigned seq = 0;
   unsigned* error = nullptr;
   int gemm_blocks = 0;
+  int flag_count = 0;  // written by every call, whatever its block shape
 };
 // Two rows a trailing block (256 blocks for 512 rows): the 512-token pass
 // at 4.59 ms against 4.60 with 4 rows, 4.61 with 8 or 1, and 4.65 with the
@@ -811,9 +812,13 @@ __global__ void Q8GemmKernel(const std::uint8_t* __restrict__ codes,
       }
       __builtin_amdgcn_s_waitcnt(WaitVm(0));
       __syncthreads();
+      // The flags past this launch's blocks take `seq` too: a call of other
+      // rows may have more blocks, and must not find its own value left there
+      // by an earlier call. No converter of this launch reads them.
       if (tid == 0)
-        __hip_atomic_store(tail.flags + tb * row_blocks + rb, tail.seq, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        for (int f = tb * row_blocks + rb; f < tail.flag_count; f += tail.gemm_blocks)
+          __hip_atomic_store(tail.flags + f, tail.seq, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
     } else if (kMaxima && row_max) {
       for (int i = tid; i < Shape::kTokens; i += Shape::kThreads)
         if (tok0 + i < n)
@@ -1011,6 +1016,7 @@ void LaunchGemm(const void* codes, const void* scales, int row_tiles, int nchunk
   int blocks = gemm_blocks;
   if (tail.out) {
     tail.gemm_blocks = gemm_blocks;
+    tail.flag_count = int(SwiGLUFlags(row_tiles, tokens));
     blocks += (int(tokens) + kHiddenRows - 1) / kHiddenRows;
   }
   Q8GemmKernel<kSwiGLU, Shape><<<blocks, Shape::kThreads, 0, stream>>>(

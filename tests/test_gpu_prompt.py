@@ -274,3 +274,43 @@ def test_gemm_swiglu_rows_is_gemm_then_half_rows(F, K, ns):
         scale = sc.download(np.float32, n + 1)
         assert np.array_equal(scale[:n], ws.download(np.float32, n)) and scale[n] == -1.0
     assert err.download(np.uint32, 1)[0] == 0
+
+
+@pytest.mark.parametrize("F,K,ns", [(7680, 2048, (512, 40, 512, 77, 512)),
+                                    (7680, 512, (128, 16, 100, 65)),
+                                    (192, 128, (300, 20, 300))])
+def test_gemm_swiglu_rows_two_values_in_turn(F, K, ns):
+    """Two sequence values in turn over calls of different token counts,
+    whose blocks map to the flags differently: a call leaves its value in
+    every flag (so the next one finds none of its own there), and its FP16
+    rows are the conversion of its own outputs."""
+    lib = L.lib()
+    g, u = L.q8(SEED, f"sf.g{F}", F, K), L.q8(SEED, f"sf.u{F}", F, K)
+    m = DeviceMatrix(g, F, K, interleave_with=u)
+    halves = half_tiles(m, 2 * F)
+    sizes = {lib.lfm3_q8_gemm_swiglu_flags_bytes(F, n) for n in range(1, 513)}
+    assert len(sizes) == 1
+    count = sizes.pop() // 4
+    flags = L.DeviceBuffer.of(np.zeros(count + 1, np.uint32))
+    err = L.DeviceBuffer.of(np.zeros(1, np.uint32))
+    blocks = lib.lfm3_q8_gemm_swiglu_max_blocks(F)
+    out_ld = (F + 63) // 64 * 64
+    for i, n in enumerate(ns):
+        print(f"[swiglu flags] F {F} K {K} n {n} seq {1 + i % 2}", flush=True)
+        x = L.normal(SEED, f"sf.x.{F}.{i}.{n}", n * K).reshape(n, K)
+        da, ds, lda = half_rows_gpu(x)
+        dy, rm = L.DeviceBuffer(n * F * 4), L.DeviceBuffer(blocks * n * 4)
+        out, sc = L.DeviceBuffer(n * out_ld * 2), L.DeviceBuffer(n * 4)
+        L.check(lib.lfm3_q8_gemm_swiglu_h16_rows(halves.addr, m.scales.addr, F, K, da.addr, lda,
+                                                 ds.addr, n, dy.addr, F, rm.addr, out.addr,
+                                                 out_ld, sc.addr, flags.addr, 1 + i % 2,
+                                                 err.addr, None))
+        L.synchronize()
+        left = flags.download(np.uint32, count + 1)
+        assert np.all(left[:count] == 1 + i % 2) and left[count] == 0
+        y = dy.download(np.float32, n * F).reshape(n, F)
+        wa, ws, wlda = half_rows_gpu(y)
+        assert np.array_equal(out.download(np.uint16, n * out_ld).reshape(n, out_ld)[:, :F],
+                              wa.download(np.uint16, n * wlda).reshape(n, wlda)[:, :F])
+        assert np.array_equal(sc.download(np.float32, n), ws.download(np.float32, n))
+    assert err.download(np.uint32, 1)[0] == 0
