@@ -32,7 +32,9 @@
 // its maximum, sum and unnormalized output, merged by CombineSpansKernel.
 // Where the workspace holds fewer records than spans, a block walks a group
 // of spans and folds them itself, with the merge's own expressions: the
-// result depends on the call's sizes, never on its workspace.
+// result depends on the call's sizes, never on its workspace (about 2 us a
+// span more than one long span would take: 17 rows after 900 keys take 34.9
+// us without a workspace, 28.4 as one span, 16.2 with a workspace).
 #include <algorithm>
 #include <cmath>
 
@@ -86,39 +88,73 @@ __device__ __forceinline__ float FoldOutput(float group_a, float a, SpanFold f) 
   return fmaf(group_a, f.old_weight, a * f.new_weight);
 }
 
-// The last span of its group of `per`.
-__device__ __forceinline__ bool EndsGroup(int s, int splits, int per) {
-  return (s + 1) % per == 0 || s + 1 == splits;
-}
+// The merge of a (row, head)'s records, kMergeDims outputs from d0 on:
+// bit s of `ends` marks the last span of a group. Every group's spans fold
+// in order, then the groups add against their common maximum (with `fold`
+// false every span is its own group), then the gate.
+constexpr int kMergeDims = 4;
 
-// Spans' records (S of them live) into their groups': a group's record takes
-// the place of its last span's. D outputs a record.
 template<int D>
-__device__ __forceinline__ void FoldGroups(float (&m)[kMaxSpans], float (&l)[kMaxSpans],
-                                           float (&a)[kMaxSpans][D], int splits, int per) {
-  float group_m = -INFINITY, group_l = 0.0f, group_a[D] = {};
+__device__ __forceinline__ void MergeRecords(const float* __restrict__ partial, std::size_t rows,
+                                             std::size_t rh, int d0, bool live, int splits,
+                                             bool fold, unsigned ends, float g,
+                                             float (&o)[kMergeDims]) {
+  // Every load (each span's maximum, sum and outputs) is issued before any
+  // arithmetic: one memory round trip. Records are D + 2 floats: 8-byte
+  // aligned pairs.
+  float m[kMaxSpans], l[kMaxSpans], a[kMaxSpans][kMergeDims];
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s) {
-    if (s >= splits)
-      break;
-    const SpanFold f = FoldWeights(group_m, group_l, m[s], l[s]);
+    const float* part = partial + (s * rows + rh) * (D + 2);
+    const bool on = live && s < splits;
+    const float2 ml = on ? *reinterpret_cast<const float2*>(part) : make_float2(-INFINITY, 0.0f);
+    const float2 v0 = on ? *reinterpret_cast<const float2*>(part + 2 + d0) : make_float2(0, 0);
+    const float2 v1 = on ? *reinterpret_cast<const float2*>(part + 4 + d0) : make_float2(0, 0);
+    m[s] = ml.x;
+    l[s] = ml.y;
+    a[s][0] = v0.x;
+    a[s][1] = v0.y;
+    a[s][2] = v1.x;
+    a[s][3] = v1.y;
+  }
+  if (fold) {  // uniform; a group's record takes the place of its last span's
+    float group_m = -INFINITY, group_l = 0.0f, group_a[kMergeDims] = {};
 #pragma unroll
-    for (int i = 0; i < D; ++i)
-      group_a[i] = FoldOutput(group_a[i], a[s][i], f);
-    if (EndsGroup(s, splits, per)) {
-      m[s] = group_m;
-      l[s] = group_l;
-      group_m = -INFINITY;
-      group_l = 0.0f;
+    for (int s = 0; s < kMaxSpans; ++s) {
+      if (s < splits) {
+        const SpanFold f = FoldWeights(group_m, group_l, m[s], l[s]);
+        const bool end = ends >> s & 1u;
 #pragma unroll
-      for (int i = 0; i < D; ++i) {
-        a[s][i] = group_a[i];
-        group_a[i] = 0.0f;
+        for (int i = 0; i < kMergeDims; ++i) {
+          group_a[i] = FoldOutput(group_a[i], a[s][i], f);
+          a[s][i] = group_a[i];
+          group_a[i] = end ? 0.0f : group_a[i];
+        }
+        l[s] = group_l;
+        m[s] = end ? group_m : -INFINITY;
+        group_m = end ? -INFINITY : group_m;
+        group_l = end ? 0.0f : group_l;
       }
-    } else {
-      m[s] = -INFINITY;  // counted in the group's
     }
   }
+  float maximum = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < kMaxSpans; ++s)
+    maximum = fmaxf(maximum, m[s]);
+  float sum = 0.0f, acc[kMergeDims] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < kMaxSpans; ++s) {
+    if (s < splits && (ends >> s & 1u)) {
+      const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
+      sum = fmaf(l[s], w, sum);
+#pragma unroll
+      for (int i = 0; i < kMergeDims; ++i)
+        acc[i] = fmaf(a[s][i], w, acc[i]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kMergeDims; ++i)
+    o[i] = (acc[i] / sum) / (1.0f + expf(-g));
 }
 
 // Keys visible to a query at absolute position p, clipped to a span
@@ -538,107 +574,56 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
   }
 }
 
-// hip/ops.hip:1692-1709: merges key spans (base-2 maxima); one block per
-// (row, head), one thread per dimension. The spans of a group of `per` fold
-// in order, then the groups add against their common maximum.
+// hip/ops.hip:1692-1709: merges key spans (base-2 maxima) into FP32 rows; a
+// thread takes kMergeDims dimensions of one (row, head), a block several
+// heads. (One block a head, one dimension a thread, was 16384 one-wave
+// blocks for 512 rows of 32 x 64 heads: the call after 300 keys 28.6 us,
+// 22.8 here; 512 rows of 16 x 128 after 900 31.4.)
+constexpr int kCombineThreads = 256;
+
 template<int D>
-__launch_bounds__(D) __global__
+__launch_bounds__(kCombineThreads) __global__
     void CombineSpansKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                             int ldg, float* __restrict__ out, int ldo, int n, int heads,
-                            int splits, int per) {
-  const int rh = blockIdx.x, d = threadIdx.x;
-  const int row = rh / heads, head = rh % heads;
-  const std::size_t rows = std::size_t(n) * heads;
-  // Every load (each span's maximum, sum and output element, and the gate)
-  // is issued before any arithmetic: one memory round trip.
-  float m[kMaxSpans], l[kMaxSpans], a[kMaxSpans][1];
-#pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s) {
-    const float* part = partial + (s * rows + rh) * (D + 2);
-    m[s] = s < splits ? part[0] : -INFINITY;
-    l[s] = s < splits ? part[1] : 0.0f;
-    a[s][0] = s < splits ? part[2 + d] : 0.0f;
-  }
-  const float g = gate[std::size_t(row) * ldg + head];
-  if (per > 1)
-    FoldGroups(m, l, a, splits, per);
-  float maximum = -INFINITY;
-#pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s)
-    maximum = fmaxf(maximum, m[s]);
-  float sum = 0.0f, acc = 0.0f;
-#pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s) {
-    if (s < splits && EndsGroup(s, splits, per)) {
-      const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
-      sum = fmaf(l[s], w, sum);
-      acc = fmaf(a[s][0], w, acc);
-    }
-  }
-  out[std::size_t(row) * ldo + head * D + d] = (acc / sum) / (1.0f + expf(-g));
+                            int splits, bool fold, unsigned ends) {
+  constexpr int kPerHead = D / kMergeDims;
+  const std::size_t t = std::size_t(blockIdx.x) * kCombineThreads + threadIdx.x;
+  const std::size_t rows = std::size_t(n) * heads, rh = t / kPerHead;
+  if (rh >= rows)
+    return;
+  const int row = int(rh / heads), head = int(rh % heads);
+  const int d0 = int(t % kPerHead) * kMergeDims;
+  float o[kMergeDims];
+  MergeRecords<D>(partial, rows, rh, d0, true, splits, fold, ends,
+                  gate[std::size_t(row) * ldg + head], o);
+  *reinterpret_cast<float4*>(out + std::size_t(row) * ldo + head * D + d0) =
+      make_float4(o[0], o[1], o[2], o[3]);
 }
 
 // The span merge of one query row over all its heads, fused with the FP16
 // row-scaled activations of the attention output (the output projection's
-// GEMM input, hip/q8_prefill.hpp:27-51): a thread takes 4 dimensions of one
-// head, merges the spans with CombineSpansKernel's expressions and order
-// (a single span reduces to the tile kernel's own (acc / sum) / (1 +
-// e^-gate)), the block reduces the row's max |out|, and the row is stored
-// as fp16(out 2^e) with scale 2^-e (HalfRowsKernel's expressions).
-constexpr int kCombineDims = 4;
-
+// GEMM input, hip/q8_prefill.hpp:27-51): CombineSpansKernel's values (a
+// single span reduces to the tile kernel's own (acc / sum) / (1 + e^-gate)),
+// the block reduces the row's max |out|, and the row is stored as
+// fp16(out 2^e) with scale 2^-e (HalfRowsKernel's expressions).
 template<int D>
 __launch_bounds__(1024) __global__
     void CombineRowsHalfKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                                int ldg, Half* __restrict__ out, int lda,
                                float* __restrict__ scale, int n, int heads, int splits,
-                               int per) {
+                               bool fold, unsigned ends) {
   __shared__ float s_max[16];
   const int row = blockIdx.x, tid = threadIdx.x;
-  constexpr int kPerHead = D / kCombineDims;
+  constexpr int kPerHead = D / kMergeDims;
   const bool live = tid < heads * kPerHead;
-  const int head = live ? tid / kPerHead : 0, d0 = (tid % kPerHead) * kCombineDims;
-  const std::size_t rh = std::size_t(row) * heads + head, rows = std::size_t(n) * heads;
-  float m[kMaxSpans], l[kMaxSpans], a[kMaxSpans][kCombineDims];
-#pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s) {
-    const float* part = partial + (s * rows + rh) * (D + 2);
-    const bool on = live && s < splits;
-    // Records are D + 2 floats: 8-byte aligned pairs.
-    const float2 ml = on ? *reinterpret_cast<const float2*>(part) : make_float2(-INFINITY, 0.0f);
-    const float2 v0 = on ? *reinterpret_cast<const float2*>(part + 2 + d0) : make_float2(0, 0);
-    const float2 v1 = on ? *reinterpret_cast<const float2*>(part + 4 + d0) : make_float2(0, 0);
-    m[s] = ml.x;
-    l[s] = ml.y;
-    a[s][0] = v0.x;
-    a[s][1] = v0.y;
-    a[s][2] = v1.x;
-    a[s][3] = v1.y;
-  }
+  const int head = live ? tid / kPerHead : 0, d0 = (tid % kPerHead) * kMergeDims;
   const float g = live ? gate[std::size_t(row) * ldg + head] : 0.0f;
-  if (per > 1)
-    FoldGroups(m, l, a, splits, per);
-  float maximum = -INFINITY;
+  float o[kMergeDims], largest = 0.0f;
+  MergeRecords<D>(partial, std::size_t(n) * heads, std::size_t(row) * heads + head, d0, live,
+                  splits, fold, ends, g, o);
 #pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s)
-    maximum = fmaxf(maximum, m[s]);
-  float sum = 0.0f, acc[kCombineDims] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < kMaxSpans; ++s) {
-    if (s < splits && EndsGroup(s, splits, per)) {
-      const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
-      sum = fmaf(l[s], w, sum);
-#pragma unroll
-      for (int i = 0; i < kCombineDims; ++i)
-        acc[i] = fmaf(a[s][i], w, acc[i]);
-    }
-  }
-  float o[kCombineDims], largest = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kCombineDims; ++i) {
-    o[i] = (acc[i] / sum) / (1.0f + expf(-g));
+  for (int i = 0; i < kMergeDims; ++i)
     largest = live ? fmaxf(largest, fabsf(o[i])) : largest;
-  }
   largest = WaveMax(largest);
   if ((tid & 63) == 0)
     s_max[tid >> 6] = largest;
@@ -739,14 +724,20 @@ void LaunchPrompt(const PromptArgs& a, hipStream_t s) {
     LaunchTiles<D, G, 2, false>(a, s);
   else
     LaunchTiles<D, G, 1, false>(a, s);
-  const int per = a.fold ? 1 : a.per;
+  // The last spans of the groups that the merge folds (all, if none).
+  const bool fold = !a.fold && a.per > 1;
+  unsigned ends = 0;
+  for (int i = 0; i < a.splits; ++i)
+    ends |= !fold || (i + 1) % a.per == 0 || i + 1 == a.splits ? 1u << i : 0u;
   if (a.out16) {
-    const int threads = (a.heads * (D / kCombineDims) + 63) / 64 * 64;
+    const int threads = (a.heads * (D / kMergeDims) + 63) / 64 * 64;
     CombineRowsHalfKernel<D><<<a.n, threads, 0, s>>>(a.partial, a.gate, a.ldg, a.out16, a.lda,
-                                                     a.scale, a.n, a.heads, a.splits, per);
+                                                     a.scale, a.n, a.heads, a.splits, fold, ends);
   } else if (a.splits > 1) {
-    CombineSpansKernel<D><<<a.n * a.heads, D, 0, s>>>(a.partial, a.gate, a.ldg, a.out, a.ldo,
-                                                       a.n, a.heads, a.splits, per);
+    const std::size_t threads = std::size_t(a.n) * a.heads * (D / kMergeDims);
+    CombineSpansKernel<D><<<unsigned((threads + kCombineThreads - 1) / kCombineThreads),
+                            kCombineThreads, 0, s>>>(a.partial, a.gate, a.ldg, a.out, a.ldo, a.n,
+                                                     a.heads, a.splits, fold, ends);
   }
 }
 
@@ -804,7 +795,7 @@ int PromptAttention(const float* q, std::uint32_t ldq, const std::uint16_t* k,
                     void* stream) {
   const std::uint32_t group = kv_heads ? heads / kv_heads : 0;
   const bool half = out16 != nullptr;
-  if (half ? (!scale || lda % kChunk || lda < heads * dim || heads * dim / kCombineDims > 1024)
+  if (half ? (!scale || lda % kChunk || lda < heads * dim || heads * dim / kMergeDims > 1024)
            : (!out || ldo < heads * dim || ldo % 4))
     return Fail(LFM3_E_INVALID, "unsupported LFM3 prompt attention output");
   if (!q || !k || !v || !gate || !rows || !heads || !kv_heads || heads % kv_heads ||
