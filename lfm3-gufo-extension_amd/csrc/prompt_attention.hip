@@ -63,10 +63,14 @@ int TileSpans(int tiles) {
   return tiles < kSplitTiles ? 1 : std::min(kMaxSpans, tiles / kSpanFloorTiles);
 }
 
-int SpanPlan(int keys, int blocks_per_span, int fill, int& span_keys) {
+// A round is an XCD's: the row blocks of a (span, KV head) pair run on one
+// XCD, the pairs on the 8 in turn. (36 pairs of 7 row blocks are 252 blocks
+// but 35 on four of the XCDs, two rounds: 400 rows after 24000 keys take 179
+// us in 9 spans, 123 in 8; 350 after 3500 58.1 in 5, 39.8 in 4.)
+int SpanPlan(int keys, int row_blocks, int kv_heads, int xcd_fill, int& span_keys) {
   const int tiles = (keys + kPAKeys - 1) / kPAKeys;
-  const int spans =
-      std::max(1, std::min(fill / std::max(blocks_per_span, 1), TileSpans(tiles)));
+  const int pairs = xcd_fill / row_blocks * 8;
+  const int spans = std::max(1, std::min(pairs / kv_heads, TileSpans(tiles)));
   span_keys = (tiles + spans - 1) / spans * kPAKeys;
   return (keys + span_keys - 1) / span_keys;
 }
@@ -679,11 +683,11 @@ int PlanSpans(int n, int position, int window, int group, int kv_heads, int dim,
     return 1;
   const int column_tiles = ColumnTiles(position, n, window, group);
   const int rows = 16 * column_tiles * kPAWaves / group;
-  const int blocks_per_span = (n + rows - 1) / rows * kv_heads;
-  // Blocks a round: two a CU where 64 dimensions and one column tile leave
-  // the registers (300 rows after 3000 of 32 x 64 heads 69.6 us against 71.4).
-  const int fill = dim == 64 && column_tiles == 1 ? 512 : 256;
-  const int spans = SpanPlan(keys, blocks_per_span, fill, span);
+  // Blocks a round of an XCD's 32 CUs: two a CU where 64 dimensions and one
+  // column tile leave the registers (300 rows after 3000 of 32 x 64 heads
+  // 69.6 us against 71.4).
+  const int xcd_fill = dim == 64 && column_tiles == 1 ? 64 : 32;
+  const int spans = SpanPlan(keys, (n + rows - 1) / rows, kv_heads, xcd_fill, span);
   if (spans == 1)
     span = keys;
   return spans;

@@ -504,6 +504,7 @@ def test_prompt_attention_span_plans(n, P, H, KH, D):
     (33, 2500, 8, 4, 128),     # few rows, two groups of five spans
     (512, 3000, 16, 4, 128),   # four spans in two groups, rows that reach the last span late
     (200, 6000, 8, 2, 64),     # a last group shorter than the others
+    (400, 5000, 16, 4, 128),   # seven row blocks, four of them a round of an XCD
 ])
 def test_prompt_attention_result_is_the_same_in_every_workspace(n, P, H, KH, D):
     """The FP32 rows bit for bit the same whatever accepted workspace they
