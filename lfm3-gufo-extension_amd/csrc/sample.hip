@@ -207,8 +207,9 @@ __device__ float BlockSum(float v, float* s_f) {
 // 17.9 here (k = 120, 4 rows: 40.3 and 23.3; k = 5: 22.0 and 13.8). What is
 // left is the two launches' latency: a slice's loads, its scan, the
 // candidates' round trip. Past kBoundMaxK the sample is too small to cut the
-// keys down, and more than kBoundMaxKeys at or above the bound (many equal
-// logits) are left to the radix select.
+// keys down, and more at or above the bound than a slice's block has threads
+// or than kBoundMaxKeys of the candidates (many equal logits) are left to the
+// radix select.
 constexpr int kBoundMaxK = 128, kBoundMaxKeys = 512;
 
 // The largest multiple t of 2^14 with at least k of the wave's keys (R a
@@ -303,10 +304,9 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
 #pragma unroll
   for (int q = 0; q < kOwn; ++q) {
     const int i = tid + kSliceThreads * q;
-    float l = raw[q];
     if (penalize && (s_bits[i >> 5] >> (i & 31) & 1u))
-      l = Penalized(l, a.penalty);
-    s_v[i] = l;
+      raw[q] = Penalized(raw[q], a.penalty);
+    s_v[i] = raw[q];
   }
   __syncthreads();
   const std::size_t unit = std::size_t(row) * slices + slice;
@@ -360,15 +360,21 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
     vals[4 * q + 3] = f.w;
   }
   if (k <= kBoundMaxK) {
-    // The bound from the threads' largest keys; the winners go out by rank,
-    // so in descending order, the lower index first where keys tie.
+    // The bound from each thread's largest key among the ones it loaded, so
+    // that a slice of few logits spreads over all threads (of its consecutive
+    // ones, 1024 logits are 64 keys, and the 64th largest of those lets
+    // through a third of the slice: 8 x 128000, whose last slice they are, at
+    // k = 64 took 32.4 us, 16.9 here). The winners go out by rank, so
+    // in descending order, the lower index first where keys tie; one a
+    // thread, as a second pass over the keys costs more than the radix
+    // select it would save (400 keys 15 us, the select 5).
     __shared__ __attribute__((aligned(16))) unsigned s_best[kSliceThreads];
-    __shared__ __attribute__((aligned(16))) unsigned s_cand[kBoundMaxKeys + 16];
-    __shared__ unsigned s_at[kBoundMaxKeys];
+    __shared__ __attribute__((aligned(16))) unsigned s_cand[kSliceThreads + 16];
+    __shared__ unsigned s_at[kSliceThreads];
     unsigned best = 0u;
 #pragma unroll
-    for (int j = 0; j < kOwn; ++j)
-      best = tid * kOwn + j < len ? max(best, OrderedBits(vals[j])) : best;
+    for (int q = 0; q < kOwn; ++q)
+      best = tid + kSliceThreads * q < len ? max(best, OrderedBits(raw[q])) : best;
     s_best[tid] = best;
     __syncthreads();
     const uint4 b4 = *reinterpret_cast<const uint4*>(&s_best[4 * (tid & 63)]);
@@ -380,7 +386,7 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
       own += tid * kOwn + j < len && OrderedBits(vals[j]) >= bound ? 1u : 0u;
     unsigned found;
     unsigned at = BlockScan<kSliceThreads>(own, s_wave, &found);
-    if (found <= unsigned(kBoundMaxKeys)) {  // uniform
+    if (found <= unsigned(kSliceThreads)) {  // uniform
       if (tid < 16)
         s_cand[found + tid] = 0u;
 #pragma unroll
@@ -394,11 +400,11 @@ __launch_bounds__(kSliceThreads) __global__ void SliceKernel(SliceArgs a) {
         }
       }
       __syncthreads();
-      for (int j = tid; j < int(found); j += kSliceThreads) {
-        const int rank = RankOf(s_cand, int(found), j);
+      if (tid < int(found)) {
+        const int rank = RankOf(s_cand, int(found), tid);
         if (rank < k) {
-          out_v[rank] = OrderedValue(s_cand[j]);
-          out_i[rank] = s_at[j];
+          out_v[rank] = OrderedValue(s_cand[tid]);
+          out_i[rank] = s_at[tid];
         }
       }
       return;

@@ -229,6 +229,10 @@ def special_rows(kind, V):
         x = -np.abs(x) - 0.5
         x[:2, ::97] = 0.0
         x[2:, ::97] = np.float32(-0.0)
+    elif kind == "leaders":    # equal leaders: as many as are ranked, one more, and beside a larger
+        for r, n in enumerate((256, 257, 512, 513)):
+            x[r, np.arange(n) * (V // 514)] = 50.0
+        x[1, V - 1] = 60.0
     elif kind == "infinite":   # masked tokens, the type's lowest value, one huge leader
         x[:, ::2] = -np.inf
         x[:, 1::6] = np.finfo(np.float32).min
@@ -236,14 +240,15 @@ def special_rows(kind, V):
     return np.ascontiguousarray(x)
 
 
-@pytest.mark.parametrize("kind", ["plain", "equal", "ties", "negative", "infinite"])
+@pytest.mark.parametrize("kind", ["plain", "equal", "ties", "negative", "infinite", "leaders"])
 @pytest.mark.parametrize("V,k", [(9000, 2), (9000, 128), (9000, 129), (4096, 64), (70000, 50),
-                                 (4200, 100)])
+                                 (4200, 100), (1000, 63), (1000, 64), (5120, 64), (4352, 128)])
 def test_top_k_edges_match_the_oracle(kind, V, k):
     """Top-k where the bounded selection starts and ends (k up to 128, at
-    most 512 keys at or above the bound, a bound above zero, slices shorter
-    than k) and where the radix select takes over: the oracle's picks over a
-    grid of uniforms."""
+    most 256 keys of a slice and 512 of the candidates at or above the
+    bound, a bound above zero, slices shorter than k and of fewer logits
+    than the block has threads or loads) and where the radix select takes
+    over: the oracle's picks over a grid of uniforms."""
     x = special_rows(kind, V)
     grid = np.linspace(0.0, 0.999, 16, dtype=np.float32)
     for r in range(x.shape[0]):
