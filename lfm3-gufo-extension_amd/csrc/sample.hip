@@ -612,18 +612,24 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   const unsigned* ci = reinterpret_cast<const unsigned*>(a.ws + a.layout.indices) +
                        std::size_t(row) * a.slices * k;
   // The candidates' keys are read from the workspace once into LDS when
-  // they fit, so the select's passes and the compaction read LDS.
-  constexpr int kStagedKeys = 8192;
-  __shared__ unsigned s_cand[kStagedKeys], s_ci[kStagedKeys];
-  const bool staged = n <= kStagedKeys;
-  if (staged) {
+  // they fit, so the select's passes and the compaction read LDS; the ranked
+  // path reads its indices there too.
+  constexpr int kStagedKeys = 8192, kRankedKeys = kSampleMaxCols / kSliceLen * kBoundMaxK;
+  static_assert(kRankedKeys <= kStagedKeys, "ranked candidates are staged");
+  __shared__ unsigned s_cand[kStagedKeys], s_ci[kRankedKeys];
+  const bool staged = n <= kStagedKeys, ranked = k <= kBoundMaxK;
+  if (ranked) {
 #pragma unroll 4
     for (int i = tid; i < n; i += kPickThreads) {
       s_cand[i] = OrderedBits(cv[i]);
       s_ci[i] = ci[i];
     }
-    __syncthreads();
+  } else if (staged) {
+#pragma unroll 4
+    for (int i = tid; i < n; i += kPickThreads)
+      s_cand[i] = OrderedBits(cv[i]);
   }
+  __syncthreads();
   const auto key_of = [&](int i) { return staged ? s_cand[i] : OrderedBits(cv[i]); };
   // Thread t owns `per` consecutive candidates (the slices' candidates in
   // slice order, so in global index order where keys tie).
@@ -633,7 +639,7 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   // bound above +0 keeps out the padding and both zeros, whose keys differ
   // though they sort as equal; ranks are then the sorted order.
   bool sorted = false;
-  if (k <= kBoundMaxK && staged) {
+  if (ranked) {
     constexpr int kSample = (2 * kBoundMaxK + kSampleMaxCols / kSliceLen + 63) / 64;
     __shared__ __attribute__((aligned(16))) unsigned s_few[kBoundMaxKeys + 16];
     __shared__ unsigned s_at[kBoundMaxKeys];
@@ -762,7 +768,7 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   }
   // The weights in parallel (the sorted maximum first), then the running
   // sums in candidate order on one thread.
-  __shared__ float s_w[kSampleMaxTopK];
+  __shared__ __attribute__((aligned(16))) float s_w[kSampleMaxTopK];
   const float top = s_val[0];
   for (int i = tid; i < k; i += kPickThreads)
     s_w[i] = expf((s_val[i] - top) * a.inv_t);
@@ -770,13 +776,30 @@ __launch_bounds__(kPickThreads) __global__ void PickKernel(PickArgs a) {
   // The running sums in candidate order on one thread (the last is the
   // total), then the first candidate with weight whose sum passes the
   // target, or the last with weight should the sums round.
-  __shared__ float s_run[kSampleMaxTopK];
+  __shared__ __attribute__((aligned(16))) float s_run[kSampleMaxTopK];
+  static_assert(kSampleMaxTopK % 16 == 0, "sixteen weights a step");
   if (tid == 0) {
     float total = 0.0f;
-#pragma unroll 8
-    for (int i = 0; i < k; ++i) {
-      total += s_w[i];
-      s_run[i] = total;
+    float4 next[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      next[q] = *reinterpret_cast<const float4*>(&s_w[4 * q]);
+    // The next sixteen weights load while these add; sums past k are not read.
+    for (int i = 0; i < k; i += 16) {
+      float4 w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[q] = next[q];
+        next[q] = *reinterpret_cast<const float4*>(&s_w[min(i + 16, kSampleMaxTopK - 16) + 4 * q]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[q].x = total += w[q].x;
+        w[q].y = total += w[q].y;
+        w[q].z = total += w[q].z;
+        w[q].w = total += w[q].w;
+        *reinterpret_cast<float4*>(&s_run[i + 4 * q]) = w[q];
+      }
     }
   }
   __syncthreads();
