@@ -145,8 +145,8 @@ int lfm3_q8_gemv_swiglu(const void* codes, const void* scales, uint32_t rows,
  * lfm3_q8_pack_host. The GEMV splits each FP32 input exactly into three
  * BF16 parts (hi + mid + lo) and each weight into one (BF16), two (F16) or
  * three (F32) BF16 parts, so that every product is exact on the BF16
- * matrix cores; sums are FP32. Any batch (decode rows in groups of 16
- * tokens; from 17 rows on, blocks of 32 or 64 tokens that split their
+ * matrix cores; sums are FP32. Any batch (groups of 16 tokens; from 17
+ * rows on, where it is faster, blocks of 32 or 64 tokens that split their
  * inputs once); cols % 32 == 0, ldx % 4 == 0, x 16-byte aligned. parts > 1
  * splits K as lfm3_q8_gemv_partials does (part p at y + p * batch * ldy);
  * lfm3_bf16_gemv_parts gives this library's choice for any float type.

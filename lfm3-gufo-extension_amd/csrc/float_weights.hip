@@ -21,10 +21,11 @@
 // 3) MFMAs per 32-column block give the exact products of the weights
 // with the FP32 inputs; only the FP32 accumulation order differs from a
 // scalar loop. Two kernels take these products. FloatGemvKernel (decode
-// rows, up to 16 tokens a block): RT row tiles a block and, per wave, a
-// contiguous range of column blocks; the waves' sums meet in LDS and add in
-// wave order. FloatGemmKernel (prompt rows): a block owns 64 tokens and
-// splits their inputs once for all of its weight rows.
+// rows, and prompt rows of few blocks; up to 16 tokens a block): RT row tiles
+// a block and, per wave, a contiguous range of column blocks; the waves' sums
+// meet in LDS and add in wave order. FloatGemmKernel (prompt rows): a block
+// owns 64 tokens (32 in the smallest shape) and splits their inputs once for
+// all of its weight rows.
 #include <cmath>
 #include <cstring>
 #include <utility>
@@ -595,6 +596,41 @@ bool PromptRows(std::uint32_t batch, std::uint32_t ldx) {
   return batch >= kGemmMinRows && BufferFits(std::size_t(batch) * ldx * 4);
 }
 
+// Calls that the prompt rows' kernel takes in blocks of 64 rows x 32 tokens:
+// where one round of them does, and up to 32 tokens.
+std::uint32_t SmallBlocks(std::uint32_t row_tiles, std::uint32_t batch) {
+  return (row_tiles + 3) / 4 * ((batch + 31) / 32);
+}
+bool TakesSmallBlocks(std::uint32_t row_tiles, std::uint32_t batch, std::uint32_t parts) {
+  return batch <= 32 || SmallBlocks(row_tiles, batch) * parts <= 256;
+}
+
+// Whether the decode rows' kernel takes prompt rows sooner: few blocks whose
+// K is not split leave the prompt kernel a long chain of steps on a part of
+// the CUs, while 16 rows x 16 tokens a block use them all. Both times in
+// microseconds, fitted to 2430 pairs of launches (BF16, F16 and F32, 256 to
+// 16384 rows, K 256 to 7680, 17 to 512 tokens, 1 to 8 parts): the kernel it
+// picks is within 0.2% of the faster on average and 29% at worst, where the
+// prompt kernel for every call was 15% slower on average. 2048 x 7680 at 17
+// tokens in one part: BF16 18.2 us against 30.7, F16 18.7 against 56.2, F32
+// 21.1 against 67.4; in 8 parts 15.9 against 8.5 (BF16). From 512 row tiles
+// on (two or four tiles a decode block) the prompt kernel won every pair. The
+// decode kernel sums a wave's products in one chain: 0.7-1.9e-7 of the result
+// from float64 for BF16 (the prompt kernel 0.8-1.4e-7), 0.9-3.4e-7 for F16
+// and F32 (0.6-1.1e-7), as decode rows have it.
+bool DecodeKernelSooner(int wf, std::uint32_t row_tiles, std::uint32_t nkb, std::uint32_t batch,
+                        std::uint32_t parts, bool swiglu) {
+  if (row_tiles >= 512 || !TakesSmallBlocks(row_tiles, batch, parts))
+    return false;
+  const double k = double(kTileCols) * nkb / parts;
+  const std::uint32_t decode =
+      (swiglu ? (row_tiles + 1) / 2 : row_tiles) * ((batch + 15) / 16) * parts;
+  const std::uint32_t rounds = (SmallBlocks(row_tiles, batch) * parts + 255) / 256;
+  const double step = wf == kBf16 ? 0.0042 : wf == kF16 ? 0.0071 : 0.0085;
+  return 2.7 + 0.0002 * k + std::max(decode, 256u) * (0.0009 + 7.9e-6 * k) <
+         rounds * (3.7 + step * k);
+}
+
 // Blocks of the prompt rows' kernel when a block owns `block_tiles` row tiles.
 std::uint32_t GemmBlocks(std::uint32_t row_tiles, std::uint32_t batch, std::uint32_t block_tiles) {
   return (row_tiles + block_tiles - 1) / block_tiles * ((batch + 63) / 64);
@@ -617,7 +653,7 @@ void GemmFormat(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, c
   const auto launch = [&](auto launcher) {
     launcher(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, parts, s);
   };
-  if (batch <= 32 || (row_tiles + 3) / 4 * ((batch + 31) / 32) * parts <= 256) {
+  if (TakesSmallBlocks(row_tiles, batch, parts)) {
     launch(LaunchGemm<2, 4, 2, kSwiGLU, WF>);
   } else if constexpr (WF == kBf16) {
     const double c[4] = {cost(32, 83.0), cost(16, 46.0), cost(8, 27.5), cost(4, 19.5)};
@@ -646,7 +682,8 @@ template<int WF>
 void LaunchFormat(const void* tiles, std::uint32_t row_tiles, std::uint32_t nkb, const float* x,
                   std::uint32_t ldx, std::uint32_t batch, float* y, std::uint32_t ldy,
                   std::uint32_t out_rows, std::uint32_t parts, bool swiglu, hipStream_t s) {
-  if (PromptRows(batch, ldx)) {
+  if (PromptRows(batch, ldx) &&
+      !DecodeKernelSooner(WF, row_tiles, nkb, batch, swiglu ? 1 : parts, swiglu)) {
     if (swiglu)
       GemmFormat<WF, true>(tiles, row_tiles, nkb, x, ldx, batch, y, ldy, out_rows, 1, s);
     else
@@ -704,14 +741,20 @@ int lfm3_float_pack_host(uint32_t type, const void* src, uint32_t rows, uint32_t
 
 uint32_t lfm3_bf16_gemv_parts(uint32_t rows, uint32_t cols, uint32_t batch) {
   // Narrow outputs split K so that the grid reaches about 256 blocks; each
-  // part keeps at least 16 column blocks (two a wave).
-  // Prompt rows count the blocks of 128 rows x 64 tokens.
+  // part keeps at least 16 column blocks (two a wave). Prompt rows count the
+  // blocks of 128 rows x 64 tokens, up to 32 of them the blocks of 64 rows x
+  // 32 tokens in parts of 8 column blocks and more: 2048 x 2048 at 17 rows
+  // with the norm that adds the parts takes 10.7 us in 8 (F16; 12.4 in 4,
+  // 11.8 unsplit), F32 12.0 (13.7, 12.5), BF16 9.8 (10.7, 11.9).
   const std::uint32_t tiles = RowTilesOf(rows);
   const std::uint32_t rt = tiles >= 1024 ? 4 : tiles >= 512 ? 2 : 1;
-  const std::uint32_t blocks =
-      batch >= kGemmMinRows ? GemmBlocks(tiles, batch, 8) : (tiles + rt - 1) / rt;
+  const bool few = batch >= kGemmMinRows && batch <= 32;
+  const std::uint32_t blocks = few                     ? SmallBlocks(tiles, batch)
+                               : batch >= kGemmMinRows ? GemmBlocks(tiles, batch, 8)
+                                                       : (tiles + rt - 1) / rt;
+  const std::uint32_t least = few ? 8 : 16;
   std::uint32_t parts = 1;
-  while (parts < 8 && blocks * parts * 2 <= 256 && ColBlocks(cols) / (parts * 2) >= 16)
+  while (parts < 8 && blocks * parts * 2 <= 256 && ColBlocks(cols) / (parts * 2) >= least)
     parts *= 2;
   return parts;
 }

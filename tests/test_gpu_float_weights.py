@@ -234,6 +234,25 @@ ALL_TYPES = dict(TYPES, bf16=L.TYPE_BF16)
 
 @pytest.mark.parametrize("kind", sorted(ALL_TYPES))
 @pytest.mark.parametrize("M,K,B,parts", [
+    (2048, 2048, 17, 1),   # few blocks of unsplit K: the decode rows' kernel
+    (2048, 2048, 17, 8),   # the same in this library's parts: the prompt rows'
+    (512, 256, 200, 1),    # a small matrix: the decode rows' kernel past one round of its blocks
+    (512, 256, 1000, 1),   # and the prompt rows' from some rows on
+    (8176, 192, 33, 1),    # 511 row tiles, the most that the decode rows' kernel takes
+    (8192, 192, 33, 1),    # 512
+])
+def test_prompt_rows_in_either_kernel(kind, M, K, B, parts):
+    """Rows that either kernel takes, at the rule's edges: against float64."""
+    tid = ALL_TYPES[kind]
+    h = synth(tid, f"fer.{kind}.{M}x{K}", M, K)
+    m, w32 = FloatMatrix(tid, h, M, K), L.float_to_f32(h, tid).reshape(M, K)
+    x = (2.0 * L.normal(SEED, f"fer.x.{M}x{K}.{B}", B * K)).reshape(B, K).astype(np.float32)
+    check_fp64(run(m, x, parts=parts), w32, x)
+    assert parts == 1 or parts == L.lib().lfm3_bf16_gemv_parts(M, K, B)
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("M,K,B,parts", [
     (1040, 160, 17, 1),    # the first batch past one token group; a part step at the end
     (8192, 64, 769, 1),    # one K group a block (512 BF16 rows), 13 token blocks, one row in the last
     (8192, 96, 385, 1),    # two K groups
