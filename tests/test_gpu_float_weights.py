@@ -253,12 +253,13 @@ def test_prompt_rows_in_either_kernel(kind, M, K, B, parts):
 
 @pytest.mark.parametrize("kind", sorted(ALL_TYPES))
 @pytest.mark.parametrize("M,K,B,parts", [
-    (1040, 160, 17, 1),    # the first batch past one token group; a part step at the end
+    (1040, 160, 17, 1),    # the first batch past one token group
     (8192, 64, 769, 1),    # one K group a block (512 BF16 rows), 13 token blocks, one row in the last
-    (8192, 96, 385, 1),    # two K groups
-    (8176, 160, 193, 1),   # four K groups, a ragged last row block
+    (8192, 96, 385, 1),    # two K groups (BF16), one (F16, F32)
+    (8176, 160, 193, 1),   # four K groups (BF16), two (F16, F32), a ragged last row block
     (48, 2048, 65, 3),     # fewer rows than a block, K parts of unequal length
-    (37, 32, 64, 1),       # one column block: three K groups have none
+    (37, 32, 64, 1),       # one column block
+    (8200, 32, 49, 1),     # one column block: three of four K groups have none
 ])
 def test_float_gemm_rows(kind, M, K, B, parts):
     """The prompt rows' kernel against float64 and, per output, against the
@@ -282,7 +283,10 @@ def test_float_gemm_swiglu(kind, F, K, B):
     """The SwiGLU epilogue over the prompt rows' kernel, in one and several
     K groups, against float64: each product within 4e-6 of its absolute sum,
     carried through y = silu(g) u (|silu'| <= 1.1, |silu(g)| <= |g|)."""
-    tid = ALL_TYPES[kind]
+    check_swiglu(ALL_TYPES[kind], kind, F, K, B)
+
+
+def check_swiglu(tid, kind, F, K, B):
     hg, hu = synth(tid, f"fgs.g.{kind}.{F}", F, K), synth(tid, f"fgs.u.{kind}.{F}", F, K)
     m = FloatMatrix(tid, None, F, K, pairs=(hg, hu))
     g32, u32 = (L.float_to_f32(h, tid).reshape(F, K) for h in (hg, hu))
@@ -293,3 +297,77 @@ def test_float_gemm_swiglu(kind, F, K, B):
     eg, eu = (4e-6 * (np.abs(x64) @ np.abs(w).T) for w in (g64, u64))
     bound = 1.1 * eg * (np.abs(u) + eu) + np.abs(g) * eu + 1e-6 * np.abs(g * u) + 1e-30
     assert np.all(np.abs(y - g / (1 + np.exp(-g)) * u) <= bound)
+
+
+# Steps of four column blocks: three whole ones and one of a single block (an
+# even number of steps), four whole and one of a single block (odd). Rows by
+# the block that GemmFormat takes for 8200 weight rows (513 or 514 row tiles,
+# which always take the prompt rows' kernel): row tiles a wave, K groups and
+# 16-token groups for BF16; for F16 and F32 where they differ.
+STEPS = [416, 544]
+BLOCKS = [17,    # <2, 4, 2>, half of its second token group empty
+          49,    # <2, 4, 4>
+          190,   # <4, 4, 4>; <2, 2, 4>
+          385,   # <4, 2, 4>; <2, 1, 4>
+          769]   # <4, 1, 4>; <2, 1, 4>
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("K", STEPS)
+@pytest.mark.parametrize("B", BLOCKS)
+def test_float_gemm_steady_state(kind, K, B):
+    """Every block shape over several whole steps and a part of one (both
+    LDS stages, the weight buffers' refill, segments that close between
+    steps, the odd last step) with a ragged last row block: against float64
+    and the decode rows' kernel."""
+    tid, M = ALL_TYPES[kind], 8200
+    h = synth(tid, f"fst.{kind}.{K}", M, K)
+    m, w32 = FloatMatrix(tid, h, M, K), L.float_to_f32(h, tid).reshape(M, K)
+    x = (2.0 * L.normal(SEED, f"fst.x.{K}.{B}", B * K)).reshape(B, K).astype(np.float32)
+    y = run(m, x)
+    check_fp64(y, w32, x)
+    scale = np.abs(x.astype(np.float64)) @ np.abs(w32.astype(np.float64)).T
+    for first in range(0, B, 64):
+        rows = np.concatenate([run(m, np.ascontiguousarray(x[i:i + 16]))
+                               for i in range(first, min(B, first + 64), 16)])
+        assert np.all(np.abs(y[first:first + 64] - rows)
+                      <= 8e-6 * scale[first:first + 64] + 1e-30)
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("F,K,B", [(4100, K, B) for K, B in zip(STEPS * 3, BLOCKS)]
+                         + [(7680, 544, 40)])
+def test_float_gemm_swiglu_steady_state(kind, F, K, B):
+    """SwiGLU in every block shape over several steps (at 40 rows of 7680
+    the smallest that takes 64 tokens): the float64 bound of the single-step
+    cases."""
+    check_swiglu(ALL_TYPES[kind], kind, F, K, B)
+
+
+@pytest.mark.parametrize("kind", sorted(ALL_TYPES))
+@pytest.mark.parametrize("B", [17, 49, 385])
+def test_float_gemm_keeps_nan_and_infinity_in_their_rows(kind, B):
+    """A NaN or infinite input reaches every output of its token and of no
+    other; a NaN or infinite weight, every output of its row and of no
+    other; all other outputs keep their bits."""
+    tid, M, K = ALL_TYPES[kind], 8200, 416
+    h = synth(tid, f"fnan.{kind}", M, K)
+    x = L.normal(SEED, f"fnan.x.{B}", B * K).reshape(B, K).astype(np.float32)
+    clean = run(FloatMatrix(tid, h, M, K), x)
+    assert np.all(np.isfinite(clean))
+    bad = x.copy()
+    bad[1, 5], bad[B - 1, K - 1] = np.nan, np.inf
+    y = run(FloatMatrix(tid, h, M, K), bad)
+    hit = np.zeros(B, bool)
+    hit[[1, B - 1]] = True
+    assert not np.isfinite(y[hit]).any()
+    assert np.array_equal(y[~hit].view(np.uint32), clean[~hit].view(np.uint32))
+    w = h.copy().reshape(M, K)
+    nan, inf = ((0x7fc0, 0x7f80) if tid == L.TYPE_BF16 else (0x7e00, 0x7c00)
+                if tid == L.TYPE_F16 else (np.nan, np.inf))
+    w[3, 400], w[M - 1, 0] = nan, inf
+    y = run(FloatMatrix(tid, w.reshape(-1), M, K), x)
+    hit = np.zeros(M, bool)
+    hit[[3, M - 1]] = True
+    assert not np.isfinite(y[:, hit]).any()
+    assert np.array_equal(y[:, ~hit].view(np.uint32), clean[:, ~hit].view(np.uint32))
