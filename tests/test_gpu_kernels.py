@@ -733,3 +733,72 @@ def test_fused_attention_group_and_ring_edges(heads, kv, D, window):
                                       True)
         ok, err = within(out[r], want)
         assert ok, (r, err)
+
+
+@pytest.mark.parametrize("heads,kv,D", [(8, 4, 64), (16, 4, 128), (16, 2, 128)])
+@pytest.mark.parametrize("positions", [(40, 700, 17), (3000, 9000, 5)])
+def test_fused_attention_keeps_nan_and_infinity_where_they_belong(heads, kv, D, positions):
+    """NaN and infinities in the decode attention, in one span and in many: a
+    query's reach its head, a value's its dimension of the heads that share
+    it, a key's every output of those heads, whether the key comes from the
+    ring or is the row's current one. Every other output keeps its bits."""
+    n, G, stride = 3, heads // kv, kv * D
+    tag = f"ann.{heads}.{kv}.{D}.{positions[0]}"
+    ld = (heads + 2 * kv) * D + heads + 4
+    k_off, v_off, g_off = heads * D, (heads + kv) * D, (heads + 2 * kv) * D
+    qkv = L.normal(SEED, tag, n * ld).reshape(n, ld)
+    qn, kn = np.ones(D, np.float32), np.ones(D, np.float32)
+    freq = np.zeros(D // 2, np.float32)      # no rotation: a query's NaN stays in its head
+    rk = [L.half_normal(SEED, f"{tag}.rk{r}", (p + 1) * stride) for r, p in enumerate(positions)]
+    rv = [L.half_normal(SEED, f"{tag}.rv{r}", (p + 1) * stride) for r, p in enumerate(positions)]
+    pos = np.array(positions, np.uint32)
+    dpos, dcap = L.DeviceBuffer.of(pos), L.DeviceBuffer.of(pos + 1)
+    dfreq, dqn, dkn = (L.DeviceBuffer.of(t) for t in (freq, qn, kn))
+    items = (L.AttentionItem * 256)()
+    count = L.check(L.lib().lfm3_attention_plan(L.ptr(pos), n, 0, items, 256))
+    ditems = L.DeviceBuffer.of(np.frombuffer(items, np.uint8, count * C_ITEM).copy())
+    ws_bytes = L.lib().lfm3_attention_workspace_bytes(count, n, heads, kv, D)
+
+    def run(qkv, rk, rv):
+        dk, dv = [L.DeviceBuffer.of(b) for b in rk], [L.DeviceBuffer.of(b) for b in rv]
+        tk, tv = pointer_table([b.addr for b in dk]), pointer_table([b.addr for b in dv])
+        dq, dout = L.DeviceBuffer.of(qkv), L.DeviceBuffer(n * heads * D * 4)
+        ws = L.DeviceBuffer.of(np.zeros(ws_bytes, np.uint8))
+        L.check(L.lib().lfm3_decode_heads_attention_ragged(
+            dq.addr, dq.addr + 4 * k_off, dq.addr + 4 * v_off, ld, dq.addr + 4 * g_off, ld,
+            dqn.addr, dkn.addr, dfreq.addr, None, tk.addr, tv.addr, dpos.addr, dcap.addr,
+            ditems.addr, count, dout.addr, heads * D, n, heads, kv, D, 1e-5, ws.addr, ws_bytes,
+            None))
+        L.synchronize()
+        return dout.download(np.float32, n * heads * D).reshape(n, heads, D)
+
+    clean = run(qkv, rk, rv)
+    assert np.all(np.isfinite(clean))
+    g = kv - 1                               # the KV head that takes the ring's bad values
+    shared = slice(g * G, (g + 1) * G)
+    for value, bits in ((np.nan, 0x7e00), (np.inf, 0x7c00)):
+        for where in ("query", "ring value", "ring key", "current value", "current key"):
+            q2, k2, v2 = qkv.copy(), [b.copy() for b in rk], [b.copy() for b in rv]
+            hit = np.zeros((n, heads, D), bool)
+            key = positions[0] // 2
+            if where == "query":
+                q2[1, 2 * D + 3] = value
+                hit[1, 2] = True
+            elif where == "ring value":
+                v2[0][key * stride + g * D + 7] = bits
+                hit[0, shared, 7] = True
+            elif where == "ring key":
+                k2[0][key * stride + g * D + 7] = bits
+                hit[0, shared] = True
+            elif where == "current value":
+                q2[2, v_off + g * D + 7] = value
+                hit[2, shared, 7] = True
+            else:
+                q2[2, k_off + g * D + 7] = value
+                hit[2, shared] = True
+            out = run(q2, k2, v2)
+            # (an infinite key whose score is -inf may also just have no weight)
+            if (where, value) != ("ring key", np.inf):
+                assert not np.isfinite(out[hit]).any(), (where, value)
+            assert np.array_equal(out[~hit].view(np.uint32), clean[~hit].view(np.uint32)), \
+                (where, value)
