@@ -976,16 +976,21 @@ int PromptParts(int row_tiles, int tokens, int nchunks) {
   return best;
 }
 
-// Each token's max |y| over 128 output columns (blockIdx.x), for the SwiGLU
-// launches whose blocks own fewer (the trailing blocks find them
-// themselves): 32 lanes a token.
+// Each token's max |y| over 128 output columns, for the SwiGLU launches whose
+// blocks own fewer (the trailing blocks find them themselves): 32 lanes a
+// token, 8 tokens a block, the token groups of a column group in turn (one
+// grid dimension: its others end at 65536 blocks, and 524288 tokens are more).
+constexpr int kMaximaTokens = 8;
+
 __global__ void RowMaximaKernel(const float* __restrict__ y, int ldy, int cols, int n,
-                                unsigned* __restrict__ row_max) {
-  const int token = blockIdx.y * 8 + int(threadIdx.x >> 5), lane = threadIdx.x & 31;
+                                int token_groups, unsigned* __restrict__ row_max) {
+  const int group = int(blockIdx.x) / token_groups;
+  const int token = int(blockIdx.x) % token_groups * kMaximaTokens + int(threadIdx.x >> 5);
+  const int lane = threadIdx.x & 31;
   float m = 0.0f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int col = blockIdx.x * 128 + 32 * j + lane;
+    const int col = group * 128 + 32 * j + lane;
     if (token < n && col < cols)
       m = fmaxf(m, fabsf(y[std::size_t(token) * ldy + col]));
   }
@@ -993,7 +998,7 @@ __global__ void RowMaximaKernel(const float* __restrict__ y, int ldy, int cols, 
   for (int k = 16; k; k >>= 1)
     m = fmaxf(m, __shfl_xor(m, k, 64));
   if (token < n && lane == 0)
-    row_max[std::size_t(blockIdx.x) * n + token] = __float_as_uint(m);
+    row_max[std::size_t(group) * n + token] = __float_as_uint(m);
 }
 
 // The kernel addresses codes, scales, activations and each output part
@@ -1024,9 +1029,11 @@ void LaunchGemm(const void* codes, const void* scales, int row_tiles, int nchunk
       nchunks, reinterpret_cast<const Half*>(a), int(lda), a_scale, int(tokens), y, int(ldy),
       int(rows), row_blocks, token_blocks, parts, part_stride, row_max, tail);
   if constexpr (kSwiGLU && !Shape::kMaxima)
-    if (row_max && !tail.out)
-      RowMaximaKernel<<<dim3((rows + 127) / 128, (tokens + 7) / 8), 256, 0, stream>>>(
-          y, int(ldy), int(rows), int(tokens), row_max);
+    if (row_max && !tail.out) {
+      const unsigned groups = (tokens + kMaximaTokens - 1) / kMaximaTokens;
+      RowMaximaKernel<<<(rows + 127) / 128 * groups, 32 * kMaximaTokens, 0, stream>>>(
+          y, int(ldy), int(rows), int(tokens), int(groups), row_max);
+    }
 }
 
 // The launcher of shape `i` (kShapeCosts) on FP16 or code tiles.

@@ -314,3 +314,16 @@ def test_gemm_swiglu_rows_two_values_in_turn(F, K, ns):
                               wa.download(np.uint16, n * wlda).reshape(n, wlda)[:, :F])
         assert np.array_equal(sc.download(np.float32, n), ws.download(np.float32, n))
     assert err.download(np.uint32, 1)[0] == 0
+
+
+def test_gemm_swiglu_row_maxima_of_many_tokens():
+    """Row maxima past 524288 tokens, of outputs narrow enough for the blocks
+    that own no 128 of them."""
+    F, K, n = 32, 32, 524303
+    g, u = L.q8(SEED, "mt.g", F, K), L.q8(SEED, "mt.u", F, K)
+    x = np.tile(L.normal(SEED, "mt.x", 4099 * K).reshape(4099, K), (128, 1))[:n]
+    y, rm = gemm(DeviceMatrix(g, F, K, interleave_with=u), x, swiglu=True, half=True)
+    assert rm.shape == (1, n)
+    assert np.array_equal(rm[0].view(np.float32), np.abs(y).max(axis=1))
+    assert np.array_equal(y[4099:8198], y[:4099])
+    assert np.all(np.isfinite(y)) and rm.any()
