@@ -139,12 +139,6 @@ __device__ __forceinline__ int XcdMajorItem(int b, int blocks) {
   return (x < rem ? x * (q + 1) : rem * (q + 1) + (x - rem) * q) + i;
 }
 
-// Per-component select (a select of whole vectors in a register array can
-// become a select of addresses into scratch memory).
-__device__ __forceinline__ uint4 SelectU4(bool p, uint4 a, uint4 b) {
-  return make_uint4(p ? a.x : b.x, p ? a.y : b.y, p ? a.z : b.z, p ? a.w : b.w);
-}
-
 // A store at kOutOfRange (or any offset past the resource) is dropped.
 __device__ __forceinline__ void StoreF32(BufferResource res, unsigned offset, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), res, offset, 0, 0);
