@@ -205,7 +205,8 @@ int lfm3_half_rows(const float* x, uint32_t ldx, const unsigned* row_max,
    in FP32), one FP32 fma per block; tokens rows of activations a (lda
    halves each, chunk tails zero) with their scales. K splits into `parts`
    (1..8) ranges written to y + p * tokens * ldy; the consumer adds the
-   parts in part order. lfm3_q8_gemm_parts gives this library's choice.
+   parts in part order. lfm3_q8_gemm_parts gives this library's choice
+   (for FP16 tiles; code tiles take any count too).
    Replaces: gpu::Project / gpu::Dense for prompt rows (LaunchSplit,
    hip/ops.hip:2019-2119; RegQ8Gemm, q8_prefill.hpp:415-645). */
 uint32_t lfm3_q8_gemm_parts(uint32_t rows, uint32_t cols, uint32_t tokens,
@@ -223,9 +224,11 @@ int lfm3_sum_parts(float* y, size_t part_stride, uint32_t rows, uint32_t cols,
                    uint32_t ld, uint32_t parts, void* stream);
 /* Gate/up over a stride-2 interleaved pair with the SwiGLU epilogue
    (q8_prefill.hpp:622-635): y = silu(g) * u, and each token row's max |y|
-   (FP32 bits) over each block of output rows stored to row_max[b * tokens
-   + t], b < lfm3_q8_gemm_swiglu_max_blocks(rows) (NULL: skipped; plain
-   stores, no zeroing needed): the partial maxima lfm3_half_rows reduces.
+   (FP32 bits) over outputs 128 b .. 128 b + 127 stored to row_max[b *
+   tokens + t], b < lfm3_q8_gemm_swiglu_max_blocks(rows), whatever block
+   shape runs (NULL: skipped; plain stores, no zeroing needed): the partial
+   maxima lfm3_half_rows reduces. Where no GEMM block owns 128 outputs a
+   second launch finds them.
    The reference forms the same row maxima with atomicMax.
    Replaces: gpu::ProjectFfn's first half for prompt rows
    (hip/ops.hip:2205-2222). */
@@ -238,10 +241,12 @@ int lfm3_q8_gemm_swiglu(const void* codes, const void* scales, uint32_t rows,
    launch: after the GEMM blocks, trailing blocks convert the SwiGLU output
    rows (y, FP32, still written) into FP16 row-scaled activations, out +
    t * out_ld with out_scale[t] (lfm3_half_rows of y with these row maxima,
-   bit for bit; chunk tails zeroed). A GEMM block writes y and its row
-   maxima through to memory and then stores `seq` in its flag; a trailing
-   block waits for the flags of its token block's GEMM blocks (bounded: a
-   timeout stores 1 to *error, which may be NULL, and the block goes on).
+   bit for bit; chunk tails zeroed). A GEMM block writes y (and the row
+   maxima of the 128 outputs it owns, if it does) through to memory and then
+   stores `seq` in its flag; a trailing block waits for the flags of its
+   token block's GEMM blocks, and writes the row maxima that no GEMM block
+   wrote (bounded: a timeout stores 1 to *error, which may be NULL, and the
+   block goes on).
    flags: lfm3_q8_gemm_swiglu_flags_bytes(rows, tokens), zeroed once; a call
    leaves `seq` in all of them (how they map to blocks depends on the token
    count). seq: nonzero and not in any of the call's flags before it: other

@@ -23,10 +23,12 @@
 // loads, and a short one the launch's fixed chain. Dropping the scores' own
 // LDS exchange, a division, two conversions a value and the current key's
 // selects, and building the query operand without a branch a read, took one
-// row of 131072 keys from 68.2 to 61.2 us (4.4 TB/s), 8 rows of 128 to 8192
-// keys from 21.0 to 19.3, 8 rows of 16K-32K from 91.6 to 88.3, 8 sliding
-// rows from 9.0 to 8.3. Eight waves a block in 128 registers: 59.2 us for
-// the one row, 102 for the eight of 16K-32K. Waves merge
+// row of 8000 keys from 28.0 to 25.5 us, of 131072 from 58.3 to 55.6 (both
+// replayed on one set of caches, partly from the memory-side cache; on
+// rotated sets 79.4 and 77.1, 3.5 TB/s), 8 rows of 128 to 8192 keys from 21.3
+// to 19.5, 8 rows of 16K-32K from 80.0 to 78.2, 8 sliding rows from 9.2 to
+// 8.4. Eight waves a block in 128 registers: 59.2 us against 61.2 for the one
+// row, 102 against 88 for the eight of 16K-32K. Waves merge
 // through LDS; rows with several spans leave per-span (max, sum, acc)
 // partials, and the last span block of a (row, KV head) to arrive merges
 // them in span order, so results do not depend on block scheduling. The

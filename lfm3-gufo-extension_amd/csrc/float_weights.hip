@@ -242,9 +242,10 @@ __device__ __forceinline__ void Unroll(F f) {
 // per 16 tokens and splits every input once per 16 RT rows, which left the
 // 512-token BF16 gate/up product (2 x 7680 x 2048) at 277-318 us; its 3 MFMAs
 // per tile, token group and 32 columns take 39 us at the matrix peak. This
-// kernel takes 79-83 us (410 TFLOP/s, 1.2 PFLOP/s of MFMAs), the down product
-// 49 us against 236, F16 gate/up 170 against 358, F32 209 against 565; what is
-// left is LDS latency at two waves a SIMD. A step of 128
+// kernel takes 85-88 us on weights from HBM (370 TFLOP/s, 1.1 PFLOP/s of
+// MFMAs; 99 at the median between a pass's other launches), the down product
+// in 2 parts 51 us against 238, F16 gate/up 185 against 369, F32 235 against
+// 575; what is left is LDS latency at two waves a SIMD. A step of 128
 // columns is split once per block into operand order in LDS (each lane's 16
 // bytes at its own slot: no bank conflicts either way), double buffered, one
 // barrier a step; each wave owns its weight rows, read straight into

@@ -27,8 +27,8 @@
 namespace lfm3amd {
 namespace {
 
-// Block shapes: WR x WT waves; each wave owns kGemmRT weight tiles (16
-// rows each) and 16 TT tokens (kGemmTT unless the shape says otherwise).
+// Block shapes: WR x WT waves; each wave owns RT weight tiles (16 rows each)
+// and 16 TT tokens (kGemmRT and kGemmTT unless the shape says otherwise).
 // The wide shape (4 x 2 waves) covers 256 weight rows and 128 tokens: 128
 // FLOP per staged byte (2 M N / (M + 2 N) for 1-byte codes and 2-byte
 // activations), about one block per CU for the 512-token pass. The narrow
@@ -76,7 +76,8 @@ using NarrowShape = GemmShape<2, 2>;
 // few tokens spends its steps waiting for memory: two chunks in flight and
 // 0.7-0.9 us a step whatever the shape. So these own 64 or 128 weight rows
 // and split their chunks over 2 to 4 K groups, which divides the steps and
-// multiplies the bytes in flight (75-150 KB of LDS, one block a CU).
+// multiplies the bytes in flight (149-151 KB of LDS on FP16 tiles, 101-124 KB
+// on code tiles: one block a CU).
 // Against the shapes they replace, alone, weights from HBM: 77 rows gate/up
 // 25.7 us (44.3), 6144 x 2048 12.3 (23.8), 2048 x 7680 in 4 parts 12.1
 // (22.9); 300 rows 6144 x 2048 19.4 (25.8); 2048 x 2048 at 200 rows in 2
@@ -234,11 +235,14 @@ __device__ __forceinline__ void BufferToLds4(BufferResource res, unsigned lane_o
 // the GEMM blocks of a launch (blockIdx.x < gemm_blocks), each further
 // block converts kHiddenRows rows of the FFN hidden output into the down
 // projection's FP16 row-scaled activations (HalfRowsKernel's expressions,
-// the row maximum from the epilogue's partial maxima). A GEMM block stores
-// its outputs and partial maxima through to memory (sc1), waits for them,
-// and then stores `seq` into its flag (flags[tb * row_blocks + rb]); a
-// converter block waits for the flags of every GEMM block of its token
-// block. The converters come after every GEMM block in dispatch order and
+// the row maximum from the partial maxima of 128 outputs each, row_max[128-row
+// block][token]). A GEMM block stores its outputs through to memory (sc1),
+// with the partial maxima where it owns 128 outputs (kMaxima), waits for them,
+// and then stores `seq` into its flag (flags[tb * row_blocks + rb]) and into
+// its share of the flags that no block of this launch has. A converter block
+// waits for the flags of every GEMM block of its token block; where no GEMM
+// block owns 128 outputs, it finds the partial maxima in the rows that it
+// holds anyway and stores them. The converters come after every GEMM block in dispatch order and
 // the GEMM blocks wait on nothing, so every wait ends; each is bounded
 // (kGemmSpinLimit polls, then error set to 1 and the block goes on).
 struct HiddenHalves {
@@ -881,8 +885,11 @@ __global__ void SumPartsKernel(float* __restrict__ y, std::size_t part_stride, i
 // launches of each shape on FP16 tiles, weights from HBM (2048 x 2048, 2048
 // x 7680, 3088 x 2048, 6144 x 2048, 20 to 512 rows, 1 to 8 parts), to within
 // 2.7 us each; the shape it picks is within 4% of the fastest on all but 12
-// of those 130 launches (where two blocks would share a CU, at most 25%).
-// The 96-row block's constants come from 18 launches at 300 to 512 rows.
+// of those 130 launches (within 25% on these).
+// The 96-row block's constants come from 18 launches at 300 to 512 rows. Code
+// tiles take the same shapes with other times: a matrix whose part count the
+// 96-row block decides can be slower there (2048 x 7680 at 640 rows in 2 parts
+// with its norm 56.8 us against 49.3 in 4; on FP16 tiles 44.8 against 52.6).
 struct ShapeCost {
   int tokens, tiles, groups;
   bool pairs;  // a wave's tiles come in gate/up pairs
