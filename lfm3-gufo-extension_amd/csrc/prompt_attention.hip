@@ -33,7 +33,7 @@
 // Where the workspace holds fewer records than spans, a block walks a group
 // of spans and folds them itself, with the merge's own expressions: the
 // result depends on the call's sizes, never on its workspace (about 2 us a
-// span more than one long span would take: 17 rows after 900 keys take 34.9
+// span more than one long span would take: 17 rows after 900 keys take 35.5
 // us without a workspace, 28.4 as one span, 16.2 with a workspace).
 #include <algorithm>
 #include <cmath>
@@ -77,7 +77,7 @@ int SpanPlan(int keys, int row_blocks, int kv_heads, int xcd_fill, int& span_key
 
 // A span's record (maximum m, sum l, output a) folded into a group's: one
 // step of the same expressions whether a block folds the spans that it walks
-// or the merge folds their records. An empty group is (-inf, 0, 0).
+// or the merge folds their records. A group's first span is its record as is.
 struct SpanFold {
   float old_weight, new_weight;
 };
@@ -121,26 +121,18 @@ __device__ __forceinline__ void MergeRecords(const float* __restrict__ partial, 
     a[s][2] = v1.x;
     a[s][3] = v1.y;
   }
-  if (fold) {  // uniform; a group's record takes the place of its last span's
-    float group_m = -INFINITY, group_l = 0.0f, group_a[kMergeDims] = {};
+  if (fold)  // uniform; a group's record ends up in its last span's place
 #pragma unroll
-    for (int s = 0; s < kMaxSpans; ++s) {
-      if (s < splits) {
+    for (int s = 1; s < kMaxSpans; ++s)
+      if (s < splits && !(ends >> (s - 1) & 1u)) {
+        float group_m = m[s - 1], group_l = l[s - 1];
         const SpanFold f = FoldWeights(group_m, group_l, m[s], l[s]);
-        const bool end = ends >> s & 1u;
-#pragma unroll
-        for (int i = 0; i < kMergeDims; ++i) {
-          group_a[i] = FoldOutput(group_a[i], a[s][i], f);
-          a[s][i] = group_a[i];
-          group_a[i] = end ? 0.0f : group_a[i];
-        }
+        m[s] = group_m;
         l[s] = group_l;
-        m[s] = end ? group_m : -INFINITY;
-        group_m = end ? -INFINITY : group_m;
-        group_l = end ? 0.0f : group_l;
+#pragma unroll
+        for (int i = 0; i < kMergeDims; ++i)
+          a[s][i] = FoldOutput(a[s - 1][i], a[s][i], f);
       }
-    }
-  }
   float maximum = -INFINITY;
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s)
@@ -480,32 +472,32 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
     }
   };
 
-  // The open span's state into the group's.
+  // The open span's state into the group's (the first one's as is).
   f4 group_acc[kFold ? CT : 1][kFold ? kDimBlocks : 1];
   float group_max[kFold ? CT : 1], group_sum[kFold ? CT : 1];
   int next_span = span_lo + sub;
-  if constexpr (kFold)
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-#pragma unroll
-      for (int m = 0; m < kDimBlocks; ++m)
-        group_acc[ct][m] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-      group_max[ct] = -INFINITY;
-      group_sum[ct] = 0.0f;
-    }
-  const auto close_span = [&]() {
+  const auto close_span = [&](bool first) {
     if constexpr (kFold)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
-        const SpanFold f = FoldWeights(group_max[ct], group_sum[ct], maximum[ct],
-                                       SumXor32(SumXor16(sum[ct])));
+        const float total = SumXor32(SumXor16(sum[ct]));
+        if (first) {  // uniform
+          group_max[ct] = maximum[ct];
+          group_sum[ct] = total;
+#pragma unroll
+          for (int m = 0; m < kDimBlocks; ++m)
+            group_acc[ct][m] = acc[ct][m];
+        } else {
+          const SpanFold f = FoldWeights(group_max[ct], group_sum[ct], maximum[ct], total);
+#pragma unroll
+          for (int m = 0; m < kDimBlocks; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              group_acc[ct][m][i] = FoldOutput(group_acc[ct][m][i], acc[ct][m][i], f);
+        }
 #pragma unroll
         for (int m = 0; m < kDimBlocks; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            group_acc[ct][m][i] = FoldOutput(group_acc[ct][m][i], acc[ct][m][i], f);
-            acc[ct][m][i] = 0.0f;
-          }
+          acc[ct][m] = f4{0.0f, 0.0f, 0.0f, 0.0f};
         maximum[ct] = -INFINITY;
         sum[ct] = 0.0f;
       }
@@ -524,7 +516,7 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
     if (base + kPAKeys <= walk.hi)
       load(base + kPAKeys);
     if (kFold && base == next_span) {
-      close_span();
+      close_span(next_span == span_lo + sub);
       next_span += sub;
     }
     if (!wave_live || base > reach.hi || base + kPAKeys <= reach.lo)
@@ -535,9 +527,9 @@ __launch_bounds__(kPAThreads) __global__ void PromptAttentionKernel(
   if constexpr (kFold) {
     // The last walked span, and those of the group past the block's rows:
     // empty records, which the merge would add too.
-    close_span();
+    close_span(next_span == span_lo + sub);
     for (; next_span <= span_hi && next_span < position + n; next_span += sub)
-      close_span();
+      close_span(false);
   }
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
