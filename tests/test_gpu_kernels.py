@@ -802,3 +802,53 @@ def test_fused_attention_keeps_nan_and_infinity_where_they_belong(heads, kv, D, 
                 assert not np.isfinite(out[hit]).any(), (where, value)
             assert np.array_equal(out[~hit].view(np.uint32), clean[~hit].view(np.uint32)), \
                 (where, value)
+
+
+@pytest.mark.parametrize("heads,kv,D", [(8, 4, 64), (16, 4, 128), (16, 2, 128)])
+@pytest.mark.parametrize("positions,window", [((200, 1500), 0), ((700, 40), 256)])
+def test_attention_weights_do_not_round_at_the_scores_size(heads, kv, D, positions, window):
+    """Scores far from zero and close together: queries and keys are small
+    integers beside one large common dimension, so every q . k is an exact
+    FP32 integer (up to 2^18) and only the weights and the sums over values
+    round. A weight e^x is then off by at most about 2^-22 (1 + |x|), |x|
+    the distance to the largest score, and those far off weigh little: the
+    outputs are within 1e-6 of the values' size. Scores rounded after the
+    scale would be off by 2^-24 of 700 (4e-5)."""
+    n, G, stride = len(positions), heads // kv, kv * D
+    tag = f"aws.{heads}.{kv}.{D}.{positions[0]}"
+    caps = [window if window else p + 1 for p in positions]
+    q = (L.uniform_u32(SEED, tag + ".q", n * heads * D, 0, 6).astype(np.float32) - 3).reshape(
+        n, heads, D)
+    q[:, :, 0] = 512.0
+    rk, rv = [], []
+    for r, c in enumerate(caps):
+        k = L.uniform_u32(SEED, f"{tag}.k{r}", c * stride, 0, 4).astype(np.float32) - 2
+        k.reshape(c, kv, D)[:, :, 0] = 16.0
+        rk.append(O.float_to_half(k))
+        rv.append(L.half_normal(SEED, f"{tag}.v{r}", c * stride))
+    gates = np.full((n, heads), 40.0, np.float32)      # 1 + e^-40 is 1
+    pos = np.array(positions, np.uint32)
+    dk, dv = [L.DeviceBuffer.of(b) for b in rk], [L.DeviceBuffer.of(b) for b in rv]
+    tk, tv = pointer_table([b.addr for b in dk]), pointer_table([b.addr for b in dv])
+    dq, dg = L.DeviceBuffer.of(q), L.DeviceBuffer.of(gates)
+    dcap = L.DeviceBuffer.of(np.array(caps, np.uint32))
+    items = (L.AttentionItem * 64)()
+    count = L.check(L.lib().lfm3_attention_plan(L.ptr(pos), n, window, items, 64))
+    ditems = L.DeviceBuffer.of(np.frombuffer(items, np.uint8, count * C_ITEM).copy())
+    ws_bytes = L.lib().lfm3_attention_workspace_bytes(count, n, heads, kv, D)
+    ws, dout = L.DeviceBuffer.of(np.zeros(ws_bytes, np.uint8)), L.DeviceBuffer(n * heads * D * 4)
+    L.check(L.lib().lfm3_decode_attention_ragged(
+        dq.addr, heads * D, dg.addr, heads, tk.addr, tv.addr, dcap.addr, ditems.addr, count,
+        dout.addr, heads * D, n, heads, kv, D, ws.addr, ws_bytes, None))
+    L.synchronize()
+    out = dout.download(np.float32, n * heads * D).reshape(n, heads, D)
+    for r, p in enumerate(positions):
+        slots = np.arange(max(0, p + 1 - window) if window else 0, p + 1) % caps[r]
+        k = O.half_to_float(rk[r]).reshape(-1, kv, D)[slots].astype(np.float64)
+        v = O.half_to_float(rv[r]).reshape(-1, kv, D)[slots].astype(np.float64)
+        for h in range(heads):
+            s = k[:, h // G] @ q[r, h].astype(np.float64) / np.sqrt(D)
+            assert s.min() > 600
+            w = np.exp(s - s.max())
+            want = (w / w.sum()) @ v[:, h // G]
+            assert np.max(np.abs(out[r, h] - want)) < 1e-6 * np.abs(v).max(), (r, h)
