@@ -92,16 +92,16 @@ __device__ __forceinline__ float FoldOutput(float group_a, float a, SpanFold f) 
   return fmaf(group_a, f.old_weight, a * f.new_weight);
 }
 
-// The merge of a (row, head)'s records, kMergeDims outputs from d0 on:
-// bit s of `ends` marks the last span of a group. Every group's spans fold
-// in order, then the groups add against their common maximum (with `fold`
-// false every span is its own group), then the gate.
+// The merge of a (row, head)'s records, kMergeDims outputs from d0 on: bit s
+// of `joins` marks a span that joins the group of the span before it, bit s
+// of `ends` the last span of a group. Every group's spans fold in order, then
+// the groups add against their common maximum, then the gate.
 constexpr int kMergeDims = 4;
 
 template<int D>
 __device__ __forceinline__ void MergeRecords(const float* __restrict__ partial, std::size_t rows,
                                              std::size_t rh, int d0, bool live, int splits,
-                                             bool fold, unsigned ends, float g,
+                                             unsigned joins, unsigned ends, float g,
                                              float (&o)[kMergeDims]) {
   // Every load (each span's maximum, sum and outputs) is issued before any
   // arithmetic: one memory round trip. Records are D + 2 floats: 8-byte
@@ -121,10 +121,10 @@ __device__ __forceinline__ void MergeRecords(const float* __restrict__ partial, 
     a[s][2] = v1.x;
     a[s][3] = v1.y;
   }
-  if (fold)  // uniform; a group's record ends up in its last span's place
+  if (joins)  // uniform; a group's record ends up in its last span's place
 #pragma unroll
     for (int s = 1; s < kMaxSpans; ++s)
-      if (s < splits && !(ends >> (s - 1) & 1u)) {
+      if (joins >> s & 1u) {
         float group_m = m[s - 1], group_l = l[s - 1];
         const SpanFold f = FoldWeights(group_m, group_l, m[s], l[s]);
         m[s] = group_m;
@@ -140,7 +140,7 @@ __device__ __forceinline__ void MergeRecords(const float* __restrict__ partial, 
   float sum = 0.0f, acc[kMergeDims] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int s = 0; s < kMaxSpans; ++s) {
-    if (s < splits && (ends >> s & 1u)) {
+    if (ends >> s & 1u) {
       const float w = __builtin_amdgcn_exp2f(m[s] - maximum);
       sum = fmaf(l[s], w, sum);
 #pragma unroll
@@ -581,7 +581,7 @@ template<int D>
 __launch_bounds__(kCombineThreads) __global__
     void CombineSpansKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                             int ldg, float* __restrict__ out, int ldo, int n, int heads,
-                            int splits, bool fold, unsigned ends) {
+                            int splits, unsigned joins, unsigned ends) {
   constexpr int kPerHead = D / kMergeDims;
   const std::size_t t = std::size_t(blockIdx.x) * kCombineThreads + threadIdx.x;
   const std::size_t rows = std::size_t(n) * heads, rh = t / kPerHead;
@@ -590,7 +590,7 @@ __launch_bounds__(kCombineThreads) __global__
   const int row = int(rh / heads), head = int(rh % heads);
   const int d0 = int(t % kPerHead) * kMergeDims;
   float o[kMergeDims];
-  MergeRecords<D>(partial, rows, rh, d0, true, splits, fold, ends,
+  MergeRecords<D>(partial, rows, rh, d0, true, splits, joins, ends,
                   gate[std::size_t(row) * ldg + head], o);
   *reinterpret_cast<float4*>(out + std::size_t(row) * ldo + head * D + d0) =
       make_float4(o[0], o[1], o[2], o[3]);
@@ -607,7 +607,7 @@ __launch_bounds__(1024) __global__
     void CombineRowsHalfKernel(const float* __restrict__ partial, const float* __restrict__ gate,
                                int ldg, Half* __restrict__ out, int lda,
                                float* __restrict__ scale, int n, int heads, int splits,
-                               bool fold, unsigned ends) {
+                               unsigned joins, unsigned ends) {
   __shared__ float s_max[16];
   const int row = blockIdx.x, tid = threadIdx.x;
   constexpr int kPerHead = D / kMergeDims;
@@ -616,7 +616,7 @@ __launch_bounds__(1024) __global__
   const float g = live ? gate[std::size_t(row) * ldg + head] : 0.0f;
   float o[kMergeDims], largest = 0.0f;
   MergeRecords<D>(partial, std::size_t(n) * heads, std::size_t(row) * heads + head, d0, live,
-                  splits, fold, ends, g, o);
+                  splits, joins, ends, g, o);
 #pragma unroll
   for (int i = 0; i < kMergeDims; ++i)
     largest = live ? fmaxf(largest, fabsf(o[i])) : largest;
@@ -720,20 +720,22 @@ void LaunchPrompt(const PromptArgs& a, hipStream_t s) {
     LaunchTiles<D, G, 2, false>(a, s);
   else
     LaunchTiles<D, G, 1, false>(a, s);
-  // The last spans of the groups that the merge folds (all, if none).
-  const bool fold = !a.fold && a.per > 1;
-  unsigned ends = 0;
-  for (int i = 0; i < a.splits; ++i)
-    ends |= !fold || (i + 1) % a.per == 0 || i + 1 == a.splits ? 1u << i : 0u;
+  // The groups that the merge folds (every record its own where a block did).
+  const int per = a.fold ? 1 : a.per;
+  unsigned joins = 0, ends = 0;
+  for (int i = 0; i < a.splits; ++i) {
+    joins |= i % per ? 1u << i : 0u;
+    ends |= (i + 1) % per == 0 || i + 1 == a.splits ? 1u << i : 0u;
+  }
   if (a.out16) {
     const int threads = (a.heads * (D / kMergeDims) + 63) / 64 * 64;
     CombineRowsHalfKernel<D><<<a.n, threads, 0, s>>>(a.partial, a.gate, a.ldg, a.out16, a.lda,
-                                                     a.scale, a.n, a.heads, a.splits, fold, ends);
+                                                     a.scale, a.n, a.heads, a.splits, joins, ends);
   } else if (a.splits > 1) {
     const std::size_t threads = std::size_t(a.n) * a.heads * (D / kMergeDims);
     CombineSpansKernel<D><<<unsigned((threads + kCombineThreads - 1) / kCombineThreads),
                             kCombineThreads, 0, s>>>(a.partial, a.gate, a.ldg, a.out, a.ldo, a.n,
-                                                     a.heads, a.splits, fold, ends);
+                                                     a.heads, a.splits, joins, ends);
   }
 }
 
